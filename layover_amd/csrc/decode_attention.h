@@ -109,6 +109,7 @@ struct DecodeArgs {
     uint32_t order;        // workgroup order, see decode_unit_of
     uint32_t vector_combine;  // workspace and out aligned for combine_dim128's vector accesses
     uint32_t shared_blocks;   // LK_DECODE_SHARED_BLOCKS: the cached form of the tile loads
+    uint32_t slots_inverse;   // ceil(2^32 / slots), for slots above 1 (decode_split_tiles)
     uint64_t block_bytes;  // bytes from one pool block to the next
     float scale_log2;      // softmax scale * log2(e)
     // Fused decode-time write (lk_paged_decode_append; null write_block: none): row b's new

@@ -76,7 +76,11 @@ struct Geometry {
     uint32_t bps;
     uint32_t splits;
     bool fast;
+    bool tiled;
 };
+
+// decode_tiles.hip
+void launch_split_tiles(const DecodeArgs& a, int kv, int qf, hipStream_t stream);
 
 uint32_t env_order() {
     static const uint32_t value = [] {
@@ -142,6 +146,13 @@ bool fast_decode(const lk_decode_shape& s, const void* pool) {
 }
 
 uint32_t compute_units();
+
+// The tiled kernel (decode_tiles.h) takes every other head_dim that is a multiple of 8 (check_shape
+// bounds it at 256), whatever the block size and formats, and needs 4-byte aligned rows, which a
+// 4-byte aligned pool gives.
+bool tiled_decode(const lk_decode_shape& s, const void* q, const void* pool) {
+    return s.head_dim % 8 == 0 && s.head_dim <= kMaxGenericDim && aligned(q, 4) && aligned(pool, 4);
+}
 
 Geometry geometry(const lk_decode_shape& s, const void* pool = nullptr) {
     Geometry g{};
@@ -240,6 +251,8 @@ void launch_decode(const DecodeArgs& a, const Geometry& g, int kv, void* out, hi
         require(grid <= 0x7FFFFFFFull, "decode grid too large");
         if (kv == LK_BF16) launch_split_mfma<LK_BF16, QF>(a, uint32_t(grid), stream);
         else launch_split_mfma<LK_FP8_RECORD, QF>(a, uint32_t(grid), stream);
+    } else if (g.tiled) {
+        launch_split_tiles(a, kv, QF, stream);
     } else {
         const uint64_t grid = uint64_t(a.batch) * a.query_heads * g.splits;
         require(grid <= 0x7FFFFFFFull, "decode grid too large");
@@ -563,7 +576,8 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     require(q && pool && table && lengths && out && workspace, "null q, pool, table, lengths, out or workspace");
     require(workspace_bytes >= ::lk::workspace_bytes(s), "workspace smaller than lk_paged_decode_workspace");
     require(aligned(workspace, 4), "workspace must be 4-byte aligned");
-    const Geometry g = geometry(s, pool);
+    Geometry g = geometry(s, pool);
+    g.tiled = !g.fast && tiled_decode(s, q, pool);
     DecodeArgs a{};
     a.q = q;
     a.pool = static_cast<const uint8_t*>(pool);
@@ -588,6 +602,7 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     a.order = env_order();
     a.shared_blocks = (s.flags & LK_DECODE_SHARED_BLOCKS) != 0;
     a.vector_combine = aligned(workspace, 16) && aligned(out, s.q_format == LK_BF16 ? 8 : 16);
+    a.slots_inverse = s.slots > 1 ? uint32_t(((1ull << 32) + s.slots - 1) / s.slots) : 0;
     a.block_bytes = pool_block_bytes(s);
     a.scale_log2 = s.scale * kLog2e;
     // One split per row (tables of at most `bps` blocks) on a grid small enough for 8-wave
@@ -595,6 +610,7 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     // which measurably costs the large-batch loop.) LAYOVER_DECODE_COMBINE keeps the combine
     // launch (for comparisons).
     if (g.fast && g.splits == 1 && env_combine() == 0 && decode_waves(a, uint64_t(s.batch) * s.kv_heads) == 8) a.out = out;
+    if (g.tiled && g.splits == 1 && env_combine() == 0) a.out = out;
     require(aligned(pool, s.kv_format == LK_F32 ? 4 : (s.kv_format == LK_BF16 ? 2 : 1)), "misaligned pool");
     if (write != nullptr) {
         require(write->write_block && write->write_slot && write->k && write->v, "null write rows, k or v");
