@@ -155,6 +155,7 @@ __device__ __forceinline__ uint32_t blocks_of(int32_t length, uint32_t slots) { 
 constexpr uint32_t kSlots = 16;
 constexpr uint32_t kDim = 128;
 constexpr uint32_t kMaxHeads = 16;  // query heads per KV head the MFMA tile holds
+constexpr uint32_t kTileTokens = 16;  // tokens per tile of the tiled kernel (decode_tiles.h)
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));

@@ -16,12 +16,15 @@
 //   steps: the k index 8g + i of the first is token 4g + i's first part for i < 4 and its second for
 //   i >= 4; the other step takes the third.
 //   FP32 queries or pools: v_mfma_f32_16x16x4_f32 throughout, FP32 as it stands.
-// Rows of tokens past the split or the sequence, and dims past head_dim, are read from a row of
-// zeros instead, so the loads need no branches and a zero weight never meets a NaN.
+// Rows of tokens past the split or the sequence are read from a row of zeros instead, so the loads
+// need no branches and a zero weight never meets a NaN.
 //
-// Measured on MI355X against one wave per (sequence, query head, split) walking its tokens one at
-// a time (the kernel below, which keeps the shapes that fit neither):
-//   see the table at launch_split_tiles in kernels.hip.
+// Measured on MI355X, per layer, against one wave per (sequence, query head, split) walking its
+// tokens one at a time (decode_split_generic, which keeps head_dims that are no multiple of 8 and
+// odd alignments): FP32 pool, 32 query heads of 128 dims, batch 4 at 700-2,500 tokens 517 -> 19 us
+// (3.4 TB/s of K and V); BF16, 64 dims, batch 16 at 300-6,000 tokens 908 -> 25 us (3.9 TB/s), the
+// merge launch apart. About 6 us of that is the chain from the launch to the first tile and from
+// the last to the partials; at long contexts the loads set the pace.
 #ifndef LAYOVER_AMD_DECODE_TILES_H
 #define LAYOVER_AMD_DECODE_TILES_H
 
@@ -31,7 +34,6 @@
 
 namespace lk {
 
-constexpr uint32_t kTileTokens = 16;
 constexpr uint32_t kTilesMaxDim = 256;
 
 // Stands for a zero part of a weight (see the weights' parts below): 2^-120 of a value is nothing.
@@ -110,7 +112,8 @@ __device__ __forceinline__ uint32_t scaled_fp8_pair(uint32_t word, bool high, in
     return bits_of(codes.x) >> 16 | bits_of(codes.y);
 }
 
-template <int KV, int QF, int kD>
+// kWhole: head_dim is kD itself.
+template <int KV, int QF, int kD, bool kWhole>
 __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 : 512) void decode_split_tiles(DecodeArgs a) {
     using Shape = TileShape<KV, QF, kD>;
     using Tile = TokenTile<KV, QF, kD>;
@@ -133,26 +136,29 @@ __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 :
     const uint32_t head0 = kv_head * a.groups + (unit % chunks) * kMaxHeads;  // first query head
     const uint32_t heads = min(kMaxHeads, a.groups - (unit % chunks) * kMaxHeads);
 
-    const int32_t length = a.lengths[uint64_t(seq) * a.lengths_stride];
-    const uint32_t nblocks = blocks_of(length, a.slots);
+    // The ids (and FP8 shifts) are loaded before the length is known, bounded by the table alone.
     const uint32_t first = split * a.bps;
-    const bool writes_out = a.out != nullptr;
-    if (first >= nblocks && !writes_out) return;
-    const uint32_t count = first < nblocks ? min(a.bps, nblocks - first) : 0;
-    const uint32_t tokens = min(uint32_t(length) - first * a.slots, count * a.slots);  // of this split
-
+    const uint32_t listed = min(a.bps, a.table_width - first);
     const uint64_t head_tile = uint64_t(a.layer) * a.kv_heads + kv_head;
     const uint64_t v_group = uint64_t(a.layers) * a.kv_heads + head_tile;
     const uint64_t group_elems = uint64_t(a.slots) * a.head_dim;
     const uint64_t block_elems = 2ull * a.layers * a.kv_heads * group_elems;
     uint32_t* s_ids = lds_words;
     uint32_t* s_shifts = lds_words + a.bps;
-    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x) {
-        const uint32_t id = uint32_t(a.table[uint64_t(seq) * a.table_stride + first + i]);
-        s_ids[i] = id;
+    const int32_t* row_ids = a.table + uint64_t(seq) * a.table_stride + first;
+    const int32_t my_id = row_ids[threadIdx.x < listed ? threadIdx.x : 0];
+    const int32_t length = a.lengths[uint64_t(seq) * a.lengths_stride];
+    const uint32_t nblocks = blocks_of(length, a.slots);
+    const bool writes_out = a.out != nullptr;
+    if (first >= nblocks && !writes_out) return;
+    const uint32_t count = first < nblocks ? min(a.bps, nblocks - first) : 0;
+    const uint32_t tokens = min(uint32_t(length) - first * a.slots, count * a.slots);  // of this split
+    // At most 256 ids and at least 256 threads.
+    if (threadIdx.x < count) {
+        s_ids[threadIdx.x] = uint32_t(my_id);
         if constexpr (KV == LK_FP8_RECORD) {
-            const uint16_t* shifts = reinterpret_cast<const uint16_t*>(a.pool + uint64_t(id) * a.block_bytes + block_elems);
-            s_shifts[i] = uint32_t(shifts[head_tile]) | uint32_t(shifts[v_group]) << 16;
+            const uint16_t* shifts = reinterpret_cast<const uint16_t*>(a.pool + uint64_t(uint32_t(my_id)) * a.block_bytes + block_elems);
+            s_shifts[threadIdx.x] = uint32_t(shifts[head_tile]) | uint32_t(shifts[v_group]) << 16;
         }
     }
 
@@ -192,33 +198,43 @@ __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 :
     // below 2^18 and slots at most 1,024, so the rounded-up reciprocal is exact).
     auto block_of = [&](uint32_t token) __attribute__((always_inline)) { return a.slots == 1 ? token : __umulhi(token, a.slots_inverse); };
 
-    auto fetch = [&](Tile& tile, uint32_t i) __attribute__((always_inline)) {
-        const uint32_t token0 = kTileTokens * (wave + i * waves);
-        const uint32_t limit = i < mine ? tokens : 0;
-        {
-            const uint32_t token = token0 + n, safe = token < limit ? token : 0;
-            const uint32_t block = block_of(safe), slot = safe - block * a.slots;
-            const uint8_t* row = a.pool + uint64_t(s_ids[block]) * a.block_bytes + (k_base + slot * row_bytes);
-            row = token < limit ? row : zeros;
-            if constexpr (KV == LK_FP8_RECORD) tile.k_shift = int32_t(int16_t(uint16_t(s_shifts[block])));
+    // Row of token n of a tile (K, then V): lane (g, n) finds it, the V loads take their four
+    // tokens' from the lanes that have them. The addresses are made opaque so that the choice
+    // between a row and the zeros stays a select.
+    const uint64_t zeros_at = reinterpret_cast<uint64_t>(zeros);
+    uint32_t from_lane[4];
 #pragma unroll
-            for (uint32_t j = 0; j < kSteps; ++j) {
-                const uint32_t dim = 4 * kChunk * j + kChunk * g;
-                load_words<kChunk * kElem>(tile.k[j], dim < a.head_dim ? row + dim * kElem : zeros);
-            }
+    for (uint32_t r = 0; r < 4; ++r) from_lane[r] = 4 * (4 * g + r);
+    // Dims past head_dim: their lanes read dims that exist instead; K's are masked off when used, V's
+    // make outputs that nothing stores.
+    auto dim_of = [&](uint32_t dim) __attribute__((always_inline)) { return kWhole || dim < a.head_dim ? dim : 0; };
+    auto fetch = [&](Tile& tile, uint32_t i) __attribute__((always_inline)) {
+        const uint32_t token = kTileTokens * (wave + i * waves) + n;
+        const bool live = i < mine && token < tokens;
+        const uint32_t safe = live ? token : 0;
+        const uint32_t block = block_of(safe), slot = safe - block * a.slots;
+        uint64_t k_row = reinterpret_cast<uint64_t>(a.pool) + uint64_t(s_ids[block]) * a.block_bytes + (k_base + slot * row_bytes);
+        uint64_t v_row = k_row + (v_base - k_base);
+        asm volatile("" : "+v"(k_row), "+v"(v_row));
+        k_row = live ? k_row : zeros_at;
+        v_row = live ? v_row : zeros_at;
+        uint32_t packed_shifts = 0;
+        if constexpr (KV == LK_FP8_RECORD) {
+            packed_shifts = s_shifts[block];
+            tile.k_shift = int32_t(int16_t(uint16_t(packed_shifts)));
         }
+        const uint8_t* k_at = reinterpret_cast<const uint8_t*>(k_row);
+#pragma unroll
+        for (uint32_t j = 0; j < kSteps; ++j) load_words<kChunk * kElem>(tile.k[j], k_at + dim_of(4 * kChunk * j + kChunk * g) * kElem);
 #pragma unroll
         for (uint32_t r = 0; r < 4; ++r) {
-            const uint32_t token = token0 + 4 * g + r, safe = token < limit ? token : 0;
-            const uint32_t block = block_of(safe), slot = safe - block * a.slots;
-            const uint8_t* row = a.pool + uint64_t(s_ids[block]) * a.block_bytes + (v_base + slot * row_bytes);
-            row = token < limit ? row : zeros;
-            if constexpr (KV == LK_FP8_RECORD) tile.shifts[r] = int32_t(s_shifts[block]);
+            const uint32_t lo = uint32_t(__builtin_amdgcn_ds_bpermute(int(from_lane[r]), int(uint32_t(v_row))));
+            const uint32_t hi = uint32_t(__builtin_amdgcn_ds_bpermute(int(from_lane[r]), int(uint32_t(v_row >> 32))));
+            const uint8_t* v_at = reinterpret_cast<const uint8_t*>(uint64_t(hi) << 32 | lo);
+            if constexpr (KV == LK_FP8_RECORD) tile.shifts[r] = __builtin_amdgcn_ds_bpermute(int(from_lane[r]), int(packed_shifts));
 #pragma unroll
-            for (uint32_t p = 0; p < Shape::kPieces; ++p) {
-                const uint32_t dim = kVDims * n + Shape::kPiece * p;
-                load_words<Shape::kPieceBytes>(tile.v[r] + p * Shape::kPieceWords, dim < a.head_dim ? row + dim * kElem : zeros);
-            }
+            for (uint32_t p = 0; p < Shape::kPieces; ++p)
+                load_words<Shape::kPieceBytes>(tile.v[r] + p * Shape::kPieceWords, v_at + dim_of(kVDims * n + Shape::kPiece * p) * kElem);
         }
     };
 
@@ -271,6 +287,13 @@ __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 :
             for (int r = 0; r < 4; ++r)
 #pragma unroll
                 for (uint32_t x = 0; x < kValueWords; ++x) vw[r][x] = tile.v[r][x];
+        }
+
+        if constexpr (!kWhole) {
+#pragma unroll
+            for (uint32_t j = 0; j < kSteps; ++j)
+#pragma unroll
+                for (int x = 0; x < 4; ++x) kb[j][x] = 4 * kChunk * j + kChunk * g < a.head_dim ? kb[j][x] : 0u;
         }
 
         f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};

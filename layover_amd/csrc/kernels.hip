@@ -6,6 +6,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <mutex>
@@ -76,11 +77,14 @@ struct Geometry {
     uint32_t bps;
     uint32_t splits;
     bool fast;
-    bool tiled;
+    uint32_t tiled;  // waves per workgroup of the tiled kernel; 0: another kernel
 };
 
+// lk_paged_decode_static's split partials, per GPU.
+constexpr uint64_t kStaticScratchBytes = 32ull << 20;
+
 // decode_tiles.hip
-void launch_split_tiles(const DecodeArgs& a, int kv, int qf, hipStream_t stream);
+void launch_split_tiles(const DecodeArgs& a, int kv, int qf, uint32_t waves, hipStream_t stream);
 
 uint32_t env_order() {
     static const uint32_t value = [] {
@@ -154,6 +158,50 @@ bool tiled_decode(const lk_decode_shape& s, const void* q, const void* pool) {
     return s.head_dim % 8 == 0 && s.head_dim <= kMaxGenericDim && aligned(q, 4) && aligned(pool, 4);
 }
 
+// Whether a shape belongs to the tiled kernel; misaligned pools of other shapes use its plan too.
+bool tiled_shape(const lk_decode_shape& s) {
+    return !(s.slots == kSlots && s.head_dim == kDim && s.kv_format != LK_F32 && s.query_heads / s.kv_heads <= kMaxHeads);
+}
+
+uint64_t partial_bytes(const lk_decode_shape& s, uint64_t splits) {
+    return uint64_t(s.batch) * s.query_heads * splits * (uint64_t(s.head_dim) + 2) * sizeof(float);
+}
+
+// Plan of the tiled kernel, in tiles of 16 tokens of one KV head (and 16 query heads): 8 waves a
+// workgroup, 4 for large launches (whose workgroups then overlap each other's ends), for more than 8
+// query heads (the merge's LDS) and for FP32 arithmetic on 256 dims (one wave per SIMD); 8 tiles a
+// wave (128 in all of 256 dims), fewer where that leaves CUs without a workgroup, at least one. Short tables
+// stay one split, which needs no merge.
+// Measured on MI355X per layer (launches in a graph, merge included):
+//   FP32, 128 dims, batch 4 at 700-2,500 tokens (20 tiles per CU), 8 waves: splits of 8, 16, 32 and 64
+//   tiles 31.3, 23.3, 28.1 and 41.7 us; 4 waves: 23.9, 29.8, 30.5 and 44.4 us
+//   BF16, 64 dims, batch 16 at 300-6,000 tokens (187 per CU), 8 waves: 16, 32, 64 and 128 tiles 40.6,
+//   32.6, 30.3 and 39.4 us; 4 waves: 32.6, 32.9, 33.3 and 40.4 us
+//   the same at batch 32 and 512-8,192 tokens (512 per CU), 8 waves: 32, 64 and 128 tiles 79.4, 78.7 and
+//   81.7 us; 4 waves, 16, 32 and 64 tiles: 76.1, 75.0 and 77.8 us; FP8 records 66.7, 64.0 and 68.1;
+//   59.2, 53.7 and 58.3 us
+//   BF16, 256 dims, 8 heads per KV head, batch 32 at 512-8,192 tokens, 4 waves: 32, 64 and 128 tiles
+//   178, 202 and 167 us; FP32, batch 16: 193, 172 and 150 us
+//   BF16, 64 dims, batch 1 at 512 tokens: 9.7 us in four splits, 7.8 us in one
+struct TiledPlan {
+    uint32_t waves, bps;
+};
+TiledPlan tiled_plan(const lk_decode_shape& s) {
+    const uint32_t groups = s.query_heads / s.kv_heads;
+    const bool wide = s.head_dim > 128;
+    const uint64_t units = uint64_t(s.batch) * s.kv_heads * ((groups + kMaxHeads - 1) / kMaxHeads);
+    const uint64_t width = (uint64_t(s.table_width) * s.slots + kTileTokens - 1) / kTileTokens;  // tiles of a full row
+    const uint64_t per_cu = (units * width + compute_units() - 1) / compute_units();
+    TiledPlan p{};
+    p.waves = groups > 8 || (wide && (s.kv_format == LK_F32 || s.q_format == LK_F32)) || per_cu >= 256 ? 4 : 8;
+    uint64_t tiles = std::max<uint64_t>(std::min<uint64_t>(wide ? 128 : 8 * p.waves, per_cu), p.waves);
+    if (width <= 4 * p.waves || (width <= 2 * tiles && units >= compute_units())) tiles = width;
+    // As many workgroups as a launch of the largest batches should have at most.
+    tiles = std::max(tiles, units * width / 65536);
+    p.bps = uint32_t(std::min<uint64_t>((tiles * kTileTokens + s.slots - 1) / s.slots, 256));
+    return p;
+}
+
 Geometry geometry(const lk_decode_shape& s, const void* pool = nullptr) {
     Geometry g{};
     g.fast = pool != nullptr && fast_decode(s, pool);
@@ -181,6 +229,12 @@ Geometry geometry(const lk_decode_shape& s, const void* pool = nullptr) {
         const uint64_t wanted = s.kv_format == LK_FP8_RECORD && s.table_width <= 64 ? 64 : std::max(large, std::min<uint64_t>(fill, 64));
         bps = 8;
         while (bps < wanted && bps < 256) bps *= 2;
+        if (tiled_shape(s)) {
+            // Partials that lk_paged_decode_static can hold, as long as the plan above keeps them so.
+            uint32_t tiled = tiled_plan(s).bps;
+            while (tiled < bps && partial_bytes(s, (s.table_width + tiled - 1) / tiled) > kStaticScratchBytes) ++tiled;
+            bps = tiled;
+        }
     }
     g.bps = bps;
     g.splits = (s.table_width + bps - 1) / bps;
@@ -202,8 +256,7 @@ void check_shape(const lk_decode_shape& s) {
 
 // Workspace: split partials, acc [batch, query_heads, splits, head_dim] then (m, l) pairs.
 uint64_t workspace_bytes(const lk_decode_shape& s) {
-    const Geometry g = geometry(s);
-    return uint64_t(s.batch) * s.query_heads * g.splits * (uint64_t(s.head_dim) + 2) * sizeof(float);
+    return partial_bytes(s, geometry(s).splits);
 }
 
 // Waves per workgroup of the matrix-core kernel: 4 when the grid gives the CUs two or more
@@ -252,7 +305,7 @@ void launch_decode(const DecodeArgs& a, const Geometry& g, int kv, void* out, hi
         if (kv == LK_BF16) launch_split_mfma<LK_BF16, QF>(a, uint32_t(grid), stream);
         else launch_split_mfma<LK_FP8_RECORD, QF>(a, uint32_t(grid), stream);
     } else if (g.tiled) {
-        launch_split_tiles(a, kv, QF, stream);
+        launch_split_tiles(a, kv, QF, g.tiled, stream);
     } else {
         const uint64_t grid = uint64_t(a.batch) * a.query_heads * g.splits;
         require(grid <= 0x7FFFFFFFull, "decode grid too large");
@@ -577,7 +630,7 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     require(workspace_bytes >= ::lk::workspace_bytes(s), "workspace smaller than lk_paged_decode_workspace");
     require(aligned(workspace, 4), "workspace must be 4-byte aligned");
     Geometry g = geometry(s, pool);
-    g.tiled = !g.fast && tiled_decode(s, q, pool);
+    g.tiled = !g.fast && tiled_decode(s, q, pool) ? tiled_plan(s).waves : 0;
     DecodeArgs a{};
     a.q = q;
     a.pool = static_cast<const uint8_t*>(pool);
@@ -673,7 +726,6 @@ LK_EXPORT int lk_paged_decode_append(const lk_decode_shape* shape, const void* q
 // caller's rule). The stream must belong to the current device, whose array is used.
 namespace lk {
 
-constexpr uint64_t kStaticScratchBytes = 32ull << 20;
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) uint8_t decode_scratch[kStaticScratchBytes];

@@ -28,7 +28,7 @@ def assembly(source: str, tmp_path: Path, *extra: str) -> str:
 
 @pytest.mark.parametrize(
     "source,extra",
-    [("kernels.hip", ()), ("prefill.hip", ("-mllvm", "--amdgpu-sched-strategy=max-ilp")), ("fp8_records.hip", ("-fgpu-flush-denormals-to-zero",))],
+    [("kernels.hip", ()), ("decode_tiles.hip", ()), ("prefill.hip", ("-mllvm", "--amdgpu-sched-strategy=max-ilp")), ("fp8_records.hip", ("-fgpu-flush-denormals-to-zero",))],
 )
 def test_kernels_use_no_scratch_spills_or_calls(source, extra, tmp_path):
     text = assembly(source, tmp_path, *extra)
