@@ -127,6 +127,11 @@ def check(status: int) -> None:
 
 
 def current_stream(device) -> int:
+    """torch's current stream on `device` as a hipStream_t. The raw query spares building a Stream
+    object, 2 us of a launch that takes 15."""
     import torch
 
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None and device.index is not None:
+        return raw(device.index)
     return torch.cuda.current_stream(device).cuda_stream

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from layover_amd.config import ModelConfig
+from layover_amd.kernels import hip_decode
 from layover_amd.kv.decode_graphs import DecodeAttentionGraphs
 from layover_amd.kv.paged_cache import BlockTable, PagedKVCache
 from oracle import oracle
@@ -257,3 +258,38 @@ def test_decode_split_plan_fills_the_gpu_at_small_batch():
     assert splits(1, 256) == 32 and splits(1, 1024) == 32 and splits(2, 256) == 16  # 8, 32, 16 blocks: 256 workgroups
     assert splits(4, 256) == 8 and splits(8, 256) == 4
     assert splits(1, 64) == 8 and splits(1, 64, _lib.LK_FP8_RECORD) == 1 and splits(1, 65, _lib.LK_FP8_RECORD) == 9
+
+
+@pytest.mark.parametrize("change", ["none", "int64_table", "strided_rows", "expanded_lengths", "narrow_stride", "q_view", "other_dtype", "layer", "kinds", "cpu"])
+def test_plain_calls_are_told_from_those_the_checks_must_see(change, monkeypatch):
+    """Only a call that validate_shapes and the layout checks would pass as it stands takes the short way
+    to the launch, and it makes the shape that decode_shape does; metadata alone decides."""
+    q, pool = torch.zeros(2, 4, 128, dtype=torch.bfloat16), torch.zeros(3, 2, 1, 2, 16, 128, dtype=torch.bfloat16)
+    packed = torch.ones(2, 8, dtype=torch.int32)
+    table, lengths, layer = packed[:, 3:], packed[:, 2], 0
+    if change == "int64_table":
+        table = table.long()
+    elif change == "strided_rows":
+        table = torch.ones(2, 10, dtype=torch.int32)[:, ::2]
+    elif change == "expanded_lengths":
+        lengths = torch.ones(1, dtype=torch.int32).expand(2)
+    elif change == "narrow_stride":
+        table = torch.ones(9, dtype=torch.int32).as_strided((2, 5), (4, 1))
+    elif change == "q_view":
+        q = torch.zeros(4, 2, 128, dtype=torch.bfloat16).transpose(0, 1)
+    elif change == "other_dtype":
+        pool = pool.half()
+    elif change == "layer":
+        layer = 1
+    elif change == "kinds":
+        pool = torch.zeros(3, 1, 1, 2, 16, 128, dtype=torch.bfloat16)
+    if change != "cpu":  # the rule looks at device numbers only
+        monkeypatch.setattr(torch.Tensor, "get_device", lambda self: 0)
+        monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    shape = hip_decode._plain_shape(q, pool, layer, table, lengths, 2, True)
+    if change != "none":
+        assert shape is None
+        return
+    expected = hip_decode.decode_shape(q, pool, layer, table, 2, lengths, True)
+    assert [getattr(shape, name) for name, _ in shape._fields_] == [getattr(expected, name) for name, _ in expected._fields_]
