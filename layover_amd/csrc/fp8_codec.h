@@ -12,8 +12,8 @@
 // Layout of work: one wave64 per group. A Qwen3-4B group (16 slots x 128 dims = 2048 values,
 // 4 KiB of BF16) is 4 loads of 16 bytes per lane, each wave instruction reading 1 KiB
 // contiguous; the shift is a wave max-reduction of the masked exponents; the 2 KiB of codes
-// go out as 4 stores of 8 bytes per lane (512 bytes contiguous per instruction). Other group
-// sizes take a strided element loop. The kernels are HBM-bound: per Qwen3-4B block, quantize
+// go out as 4 stores of 8 bytes per lane (512 bytes contiguous per instruction). Other multiples
+// of 8 values take the vector kernels of fp8_records.hip, any other size a strided element loop. The kernels are HBM-bound: per Qwen3-4B block, quantize
 // reads 2,359,296 bytes and writes 1,180,800; dequantize the reverse.
 #ifndef LAYOVER_AMD_FP8_CODEC_H
 #define LAYOVER_AMD_FP8_CODEC_H
@@ -206,6 +206,13 @@ void launch_quantize_2048(const uint16_t* pool, const int32_t* ids, uint8_t* sta
                           uint32_t grid, hipStream_t stream);
 void launch_dequantize_2048(const uint8_t* stage, const int32_t* ids, uint16_t* pool, uint32_t count, uint32_t groups_per_block,
                             uint32_t grid, hipStream_t stream);
+// Groups of any multiple of 8 values up to kVectorGroup: a 16-byte aligned pool, stage and records 4-byte
+// aligned, `total` groups (count x groups_per_block) below 2^31.
+constexpr uint32_t kVectorGroup = 4096;
+void launch_quantize_vector(const uint16_t* pool, const int32_t* ids, uint8_t* stage, uint32_t total, uint32_t group_elems,
+                            uint32_t groups_per_block, hipStream_t stream);
+void launch_dequantize_vector(const uint8_t* stage, const int32_t* ids, uint16_t* pool, uint32_t total, uint32_t group_elems,
+                              uint32_t groups_per_block, hipStream_t stream);
 // One token per row written into Qwen3-shaped FP8 records (16 slots x 128 dims, 16-byte
 // aligned records, k and v), the fast form of lk_fp8_append.
 void launch_append_2048(uint8_t* records, const int32_t* write_block, const int32_t* write_slot, uint32_t row_stride, uint32_t batch,
@@ -222,7 +229,8 @@ void launch_stage_history_2048(const uint8_t* records, const int32_t* ids, uint6
 // unit of the library.
 namespace {
 
-// Any group size and alignment: element-strided loops, one wave per group.
+// Any group size and alignment (what the kernels above do not take): element-strided loops, one wave
+// per group.
 __global__ __launch_bounds__(kWave* kCodecWaves) void quantize_groups_any(const uint16_t* __restrict__ pool, const int32_t* __restrict__ ids,
                                                                         uint8_t* __restrict__ stage, uint32_t count,
                                                                         uint64_t group_elems, uint32_t groups_per_block) {

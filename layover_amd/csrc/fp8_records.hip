@@ -28,6 +28,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "fp8_codec.h"
 
 namespace lk {
@@ -318,6 +320,190 @@ __global__ __launch_bounds__(kWave* kCodecWaves) void append_groups_2048(uint8_t
     const uint32_t g = (kind * layers + layer) * kv_heads + head;
     uint8_t* base = records + uint64_t(block) * record;
     append_group_2048(base + uint64_t(g) * kFastGroup, reinterpret_cast<int16_t*>(base + block_elems + 2ull * g), write, fresh, lane);
+}
+
+// Groups of any other size that is a multiple of 8, up to 4,096 values (kVectorGroup), 16 bytes of BF16 and 8 codes
+// a lane and load, in the same two passes over registers as the 2,048-value kernels. A group of up to
+// 512 values takes the power of two of lanes that holds it, so a wave converts 64 >> lanes_log2 groups
+// side by side (kSide); larger groups take kChunks loads a lane. kSets such sets per wave keep four
+// loads a lane in flight whatever the size, as the 2,048-value kernels have. HBM-bound: measured on
+// MI355X, 300 blocks of 24 layers x 8 heads x 1,024-value groups (16 x 64), quantize 248 us one
+// element at a time -> 58 us, dequantize 143 -> 62 us (6.1 and 5.7 TB/s of read and write).
+constexpr uint32_t kLaneValues = 8;
+typedef uint32_t codes8 __attribute__((ext_vector_type(2), aligned(4)));  // records are 4-byte aligned at least
+
+// Where lane's part of chunk c of set s lies; dead lanes point at the start of an existing group.
+struct VectorPlace {
+    uint32_t index, g, offset;
+    bool live;
+};
+template <int kSets, bool kSide>
+__device__ __forceinline__ VectorPlace vector_place(uint32_t wave, uint32_t lane, int set, int chunk, uint32_t total, uint32_t group_elems,
+                                                    uint32_t groups_per_block, uint32_t lanes_log2) {
+    VectorPlace p;
+    const uint32_t group = kSide ? ((wave * kSets + set) << (6 - lanes_log2)) + (lane >> lanes_log2) : wave * kSets + set;
+    const uint32_t within = kSide ? lane & ((1u << lanes_log2) - 1) : lane;
+    const uint32_t value = (chunk * kWave + within) * kLaneValues;
+    p.live = group < total && value < group_elems;
+    const uint32_t safe = group < total ? group : 0;
+    p.index = safe / groups_per_block;
+    p.g = safe % groups_per_block;
+    p.offset = p.live ? value : 0;
+    return p;
+}
+
+// Max over the lanes of a group (all 64, or 1 << lanes_log2 of them).
+template <bool kSide>
+__device__ __forceinline__ uint32_t group_max(uint32_t value, uint32_t lanes_log2) {
+    if constexpr (!kSide) return wave_max(value);
+    for (uint32_t mask = 1u << lanes_log2 >> 1; mask >= 1; mask >>= 1) {
+        const uint32_t other = __shfl_xor(value, int(mask), kWave);
+        value = other > value ? other : value;
+    }
+    return value;
+}
+
+template <int kChunks, int kSets, bool kSide>
+__global__ __launch_bounds__(kWave) void quantize_groups_vector(const uint16_t* __restrict__ pool, const int32_t* __restrict__ ids,
+                                                                uint8_t* __restrict__ stage, uint32_t total, uint32_t group_elems,
+                                                                uint32_t groups_per_block, uint32_t lanes_log2) {
+    const uint32_t lane = threadIdx.x;
+    const uint64_t block_elems = uint64_t(group_elems) * groups_per_block;
+    const uint64_t record = block_elems + 2ull * groups_per_block;
+    u32x4 words[kSets][kChunks];
+#pragma unroll
+    for (int s = 0; s < kSets; ++s)
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const VectorPlace p = vector_place<kSets, kSide>(blockIdx.x, lane, s, c, total, group_elems, groups_per_block, lanes_log2);
+            const uint16_t* source = pool + uint64_t(ids[p.index]) * block_elems + uint64_t(p.g) * group_elems + p.offset;
+            words[s][c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(source));
+        }
+#pragma unroll
+    for (int s = 0; s < kSets; ++s) {
+        u16x2 keys = {0, 0};
+        uint32_t flags = 0;
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const VectorPlace p = vector_place<kSets, kSide>(blockIdx.x, lane, s, c, total, group_elems, groups_per_block, lanes_log2);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const uint32_t word = p.live ? words[s][c][w] : 0u;
+                const uint32_t stepped = (word & 0x7F807F80u) + 0x00800080u;
+                flags |= stepped;
+                keys = __builtin_elementwise_max(keys, __builtin_bit_cast(u16x2, stepped & 0x7FFF7FFFu));
+            }
+        }
+        const int32_t shift = shift_from_key(group_max<kSide>(uint32_t(keys.x > keys.y ? keys.x : keys.y) >> 7, lanes_log2));
+        // The hardware convert where it is exact for every group of the wave (see the head of this file).
+        const bool plain = !__any((flags & 0x80008000u) != 0 || shift < -126);
+        const float scale = power_of_two(plain ? -shift : 0);
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const VectorPlace p = vector_place<kSets, kSide>(blockIdx.x, lane, s, c, total, group_elems, groups_per_block, lanes_log2);
+            uint32_t packed[2];
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const uint32_t a = words[s][c][2 * half], b = words[s][c][2 * half + 1];
+                if (plain) {
+                    int v = __builtin_amdgcn_cvt_pk_fp8_f32(__uint_as_float(a << 16) * scale, __uint_as_float(a & 0xFFFF0000u) * scale, 0, false);
+                    v = __builtin_amdgcn_cvt_pk_fp8_f32(__uint_as_float(b << 16) * scale, __uint_as_float(b & 0xFFFF0000u) * scale, v, true);
+                    packed[half] = uint32_t(v);
+                } else {
+                    packed[half] = encode_e4m3(a & 0xFFFFu, shift) | (encode_e4m3(a >> 16, shift) << 8) |
+                                   (encode_e4m3(b & 0xFFFFu, shift) << 16) | (encode_e4m3(b >> 16, shift) << 24);
+                }
+            }
+            uint8_t* out = stage + uint64_t(p.index) * record;
+            if (p.live) {
+                __builtin_nontemporal_store(codes8{packed[0], packed[1]}, reinterpret_cast<codes8*>(out + uint64_t(p.g) * group_elems + p.offset));
+                if (p.offset == 0) *reinterpret_cast<int16_t*>(out + block_elems + 2ull * p.g) = int16_t(shift);
+            }
+        }
+    }
+}
+
+template <int kChunks, int kSets, bool kSide>
+__global__ __launch_bounds__(kWave) void dequantize_groups_vector(const uint8_t* __restrict__ stage, const int32_t* __restrict__ ids,
+                                                                  uint16_t* __restrict__ pool, uint32_t total, uint32_t group_elems,
+                                                                  uint32_t groups_per_block, uint32_t lanes_log2) {
+    const uint32_t lane = threadIdx.x;
+    const uint64_t block_elems = uint64_t(group_elems) * groups_per_block;
+    const uint64_t record = block_elems + 2ull * groups_per_block;
+    codes8 bytes[kSets][kChunks];
+    int32_t shift[kSets];
+    uint64_t block[kSets];
+#pragma unroll
+    for (int s = 0; s < kSets; ++s)
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const VectorPlace p = vector_place<kSets, kSide>(blockIdx.x, lane, s, c, total, group_elems, groups_per_block, lanes_log2);
+            const uint8_t* in = stage + uint64_t(p.index) * record;
+            bytes[s][c] = __builtin_nontemporal_load(reinterpret_cast<const codes8*>(in + uint64_t(p.g) * group_elems + p.offset));
+            if (c == 0) {
+                shift[s] = *reinterpret_cast<const int16_t*>(in + block_elems + 2ull * p.g);
+                block[s] = uint64_t(uint32_t(ids[p.index]));
+            }
+        }
+#pragma unroll
+    for (int s = 0; s < kSets; ++s) {
+        // A byte 0x7F or 0xFF (NaN) becomes 0x80 after masking off its sign and adding one.
+        uint32_t flags = 0;
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) flags |= ((bytes[s][c][0] & 0x7F7F7F7Fu) + 0x01010101u) | ((bytes[s][c][1] & 0x7F7F7F7Fu) + 0x01010101u);
+        const bool plain = !__any((flags & 0x80808080u) != 0 || shift[s] < -117 || shift[s] > 119);
+        const float scale = power_of_two(plain ? shift[s] : 0);
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const VectorPlace p = vector_place<kSets, kSide>(blockIdx.x, lane, s, c, total, group_elems, groups_per_block, lanes_log2);
+            u32x4 out;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const uint32_t word = bytes[s][c][w / 2];
+                if (plain) {
+                    out[w] = w % 2 ? __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(word, scale, true))
+                                   : __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(word, scale, false));
+                } else {
+                    const uint32_t pair = word >> (16 * (w % 2));
+                    out[w] = decode_e4m3(pair & 0xFFu, shift[s]) | (decode_e4m3((pair >> 8) & 0xFFu, shift[s]) << 16);
+                }
+            }
+            if (p.live) __builtin_nontemporal_store(out, reinterpret_cast<u32x4*>(pool + block[s] * block_elems + uint64_t(p.g) * group_elems + p.offset));
+        }
+    }
+}
+
+// The instance for a group size, applied to (chunks, sets, side) as integral constants, and the waves
+// it needs for `total` groups.
+template <class Launch>
+static void with_vector_shape(uint32_t group_elems, uint32_t total, Launch&& launch) {
+    const uint32_t lanes = (group_elems + kLaneValues - 1) / kLaneValues;
+    uint32_t lanes_log2 = 0;
+    while ((1u << lanes_log2) < lanes && lanes_log2 < 6) ++lanes_log2;
+    const uint32_t chunks = (lanes + kWave - 1) / kWave;
+    const auto grid = [&](uint32_t per_wave) { return dim3((total + per_wave - 1) / per_wave); };
+    using std::integral_constant;
+    if (lanes_log2 < 6) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{}, std::true_type{}, grid(4u << (6 - lanes_log2)), lanes_log2);
+    else if (chunks == 1) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{}, std::false_type{}, grid(4), lanes_log2);
+    else if (chunks == 2) launch(integral_constant<int, 2>{}, integral_constant<int, 2>{}, std::false_type{}, grid(2), lanes_log2);
+    else if (chunks <= 4) launch(integral_constant<int, 4>{}, integral_constant<int, 1>{}, std::false_type{}, grid(1), lanes_log2);
+    else launch(integral_constant<int, 8>{}, integral_constant<int, 1>{}, std::false_type{}, grid(1), lanes_log2);
+}
+
+void launch_quantize_vector(const uint16_t* pool, const int32_t* ids, uint8_t* stage, uint32_t total, uint32_t group_elems,
+                            uint32_t groups_per_block, hipStream_t stream) {
+    with_vector_shape(group_elems, total, [&](auto chunks, auto sets, auto side, dim3 grid, uint32_t lanes_log2) {
+        hipLaunchKernelGGL((quantize_groups_vector<decltype(chunks)::value, decltype(sets)::value, decltype(side)::value>), grid, dim3(kWave), 0,
+                           stream, pool, ids, stage, total, group_elems, groups_per_block, lanes_log2);
+    });
+}
+
+void launch_dequantize_vector(const uint8_t* stage, const int32_t* ids, uint16_t* pool, uint32_t total, uint32_t group_elems,
+                              uint32_t groups_per_block, hipStream_t stream) {
+    with_vector_shape(group_elems, total, [&](auto chunks, auto sets, auto side, dim3 grid, uint32_t lanes_log2) {
+        hipLaunchKernelGGL((dequantize_groups_vector<decltype(chunks)::value, decltype(sets)::value, decltype(side)::value>), grid, dim3(kWave),
+                           0, stream, stage, ids, pool, total, group_elems, groups_per_block, lanes_log2);
+    });
 }
 
 void launch_append_2048(uint8_t* records, const int32_t* write_block, const int32_t* write_slot, uint32_t row_stride, uint32_t batch,

@@ -67,6 +67,13 @@ bool fast_records(const void* pool, const void* stage, uint64_t group_elems, uin
     return group_elems == kFastGroup && aligned(pool, 16) && aligned(stage, 16) && record % 16 == 0;
 }
 
+// The vector kernels take what 16-byte loads of the pool and 8-byte ones of the records (4-byte aligned)
+// can: every even number of groups a block of a multiple of 8 values, up to 4,096.
+bool vector_records(const void* pool, const void* stage, uint32_t count, uint64_t group_elems, uint32_t groups_per_block) {
+    return group_elems % 8 == 0 && group_elems <= kVectorGroup && groups_per_block % 2 == 0 && aligned(pool, 16) && aligned(stage, 4) &&
+           uint64_t(count) * groups_per_block < 0x7FFFFFFFull;
+}
+
 // Decode launch geometry: blocks per split (bps) and splits per sequence, from the shape only.
 // About 16 workgroups per CU if every row used the whole table width (so about 8 at the
 // typical half-full width of mixed lengths), with splits of 64 to 256 blocks: shorter splits
@@ -515,6 +522,9 @@ LK_EXPORT int lk_fp8_quantize(const void* pool, const int32_t* ids, uint32_t cou
         if (lk::fast_records(pool, stage, group_elems, groups_per_block))
             lk::launch_quantize_2048(static_cast<const uint16_t*>(pool), ids, static_cast<uint8_t*>(stage), count, groups_per_block,
                                      lk::codec_grid(groups), s);
+        else if (lk::vector_records(pool, stage, count, group_elems, groups_per_block))
+            lk::launch_quantize_vector(static_cast<const uint16_t*>(pool), ids, static_cast<uint8_t*>(stage), uint32_t(groups),
+                                       uint32_t(group_elems), groups_per_block, s);
         else
             hipLaunchKernelGGL(lk::quantize_groups_any, dim3(grid), block, 0, s, static_cast<const uint16_t*>(pool), ids,
                                static_cast<uint8_t*>(stage), count, group_elems, groups_per_block);
@@ -533,6 +543,9 @@ LK_EXPORT int lk_fp8_dequantize(const void* stage, const int32_t* ids, uint32_t 
         if (lk::fast_records(pool, stage, group_elems, groups_per_block))
             lk::launch_dequantize_2048(static_cast<const uint8_t*>(stage), ids, static_cast<uint16_t*>(pool), count, groups_per_block,
                                        lk::codec_grid(groups), s);
+        else if (lk::vector_records(pool, stage, count, group_elems, groups_per_block))
+            lk::launch_dequantize_vector(static_cast<const uint8_t*>(stage), ids, static_cast<uint16_t*>(pool), uint32_t(groups),
+                                         uint32_t(group_elems), groups_per_block, s);
         else
             hipLaunchKernelGGL(lk::dequantize_groups_any, dim3(grid), block, 0, s, static_cast<const uint8_t*>(stage), ids,
                                static_cast<uint16_t*>(pool), count, group_elems, groups_per_block);
