@@ -84,7 +84,7 @@ typedef struct {
     float scale;          /* softmax scale, 1/sqrt(head_dim) in the reference */
     uint32_t table_stride;   /* int32 elements between table rows; 0 means table_width */
     uint32_t lengths_stride; /* int32 elements between lengths; 0 means 1 */
-    uint32_t flags;          /* 0, or LK_DECODE_SHARED_BLOCKS */
+    uint32_t flags;          /* 0, LK_DECODE_SHARED_BLOCKS, LK_DECODE_LAYERS(count, rows) */
 } lk_decode_shape;
 
 /* Decode flag: rows of the table share pool blocks (forked prefixes, or tables drawn from a
@@ -93,6 +93,14 @@ typedef struct {
  * Cache serves the repeats). Without it the tiles are streamed with the non-temporal hint,
  * the faster form when every block is read once per layer. Results are the same either way. */
 #define LK_DECODE_SHARED_BLOCKS 1u
+
+/* Decode flag: the launch covers `count` layers (1 to 255) from shape->layer on, for callers that
+ * hold every layer's queries at once. Table and lengths (and write positions) serve all of them; q
+ * and k, v of layer i start at row i * rows of the arrays given (rows >= batch, below 65536), out is
+ * [count, batch, query_heads, head_dim] contiguous. The same results as one call per layer, up to
+ * the order in which a row's partial sums are added; the workspace is sized for the whole launch.
+ * Not for lk_paged_decode_static. */
+#define LK_DECODE_LAYERS(count, rows) (((uint32_t)(count) << 8) | ((uint32_t)(rows) << 16))
 
 /* Bytes of device workspace lk_paged_decode needs for this shape (split-K partial results).
  * Depends only on the shape and on the current device's compute-unit count (a grid too small

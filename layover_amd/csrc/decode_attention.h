@@ -103,6 +103,10 @@ struct DecodeArgs {
     uint32_t batch, query_heads, kv_heads, head_dim, layers, slots, layer, table_width;
     uint32_t table_stride;   // int32 elements from one table row to the next (>= table_width)
     uint32_t lengths_stride; // int32 elements from one length to the next
+    // Layers of one launch (grid.y; LK_DECODE_LAYERS): layer `layer + y` reads its queries and new
+    // tokens layer_rows rows further on, and its partials and outputs follow by `batch` rows.
+    uint32_t layer_count, layer_rows;
+    uint32_t waves;        // per workgroup of the split kernel
     uint32_t groups;       // query heads per KV head
     uint32_t splits;       // splits per sequence (grid)
     uint32_t bps;          // blocks per split
@@ -279,6 +283,8 @@ __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(K
     uint32_t split, kv_head, seq;
     if (!decode_unit_of(a, blockIdx.x, &seq, &split, &kv_head)) return;
     const uint32_t groups = a.groups;
+    const uint32_t layer = a.layer + blockIdx.y;
+    const uint32_t in_row = blockIdx.y * a.layer_rows + seq, out_row = blockIdx.y * a.batch + seq;
 
     // The split's block ids are loaded (one per lane, this wave's units) before the length
     // is known, bounded by the table width alone, so the two loads overlap; the length then
@@ -302,7 +308,7 @@ __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(K
 #pragma unroll
         for (int i = 0; i < 16; ++i) qt[part][i] = 0;
     if (n < groups) {
-        const uint64_t row_at = (uint64_t(seq) * a.query_heads + kv_head * groups + n) * kDim + MfmaTile<KV>::kGroupDims * g;
+        const uint64_t row_at = (uint64_t(in_row) * a.query_heads + kv_head * groups + n) * kDim + MfmaTile<KV>::kGroupDims * g;
         constexpr uint32_t kStepDims = MfmaTile<KV>::kStepDims;
         if constexpr (QF == LK_BF16) {
 #pragma unroll
@@ -337,7 +343,7 @@ __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(K
 
     constexpr uint32_t kElem = KV == LK_FP8_RECORD ? 1 : 2;
     const uint64_t tile_bytes = uint64_t(kSlots) * kDim * kElem;
-    const uint64_t head_tile = uint64_t(a.layer) * a.kv_heads + kv_head;  // group index of K
+    const uint64_t head_tile = uint64_t(layer) * a.kv_heads + kv_head;  // group index of K
     const uint64_t k_offset = head_tile * tile_bytes + (uint64_t(n) * kDim + MfmaTile<KV>::kGroupDims * g) * kElem;
     const uint64_t v_offset = (uint64_t(a.layers) * a.kv_heads + head_tile) * tile_bytes + (uint64_t(4 * g) * kDim + 8 * n) * kElem;
     const uint64_t block_elems = uint64_t(2) * a.layers * a.kv_heads * kSlots * kDim;  // FP8: shifts follow the data
@@ -380,8 +386,8 @@ __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(K
     if (wave == writer) {
         const uint32_t block = uint32_t(a.write_block[uint64_t(seq) * a.write_stride]);
         write_slot = uint32_t(a.write_slot[uint64_t(seq) * a.write_stride]);
-        const uint16_t* k_row = a.k_new + (uint64_t(seq) * a.kv_heads + kv_head) * kDim;
-        const uint16_t* v_row = a.v_new + (uint64_t(seq) * a.kv_heads + kv_head) * kDim;
+        const uint16_t* k_row = a.k_new + (uint64_t(in_row) * a.kv_heads + kv_head) * kDim;
+        const uint16_t* v_row = a.v_new + (uint64_t(in_row) * a.kv_heads + kv_head) * kDim;
         uint8_t* base = const_cast<uint8_t*>(a.pool) + uint64_t(block) * a.block_bytes;  // the pool is written only here
         const uint64_t k_group = head_tile, v_group = uint64_t(a.layers) * a.kv_heads + head_tile;
         if constexpr (kBf16) {
@@ -743,14 +749,14 @@ __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(K
             // The row's only split: the combine's arithmetic for one split (weight 1, its sum
             // starting from +0, so a -0 becomes +0 there too), times the reciprocal of l, so
             // results equal the two-launch form bit for bit.
-            const uint64_t at = (uint64_t(seq) * a.query_heads + kv_head * groups + h) * kDim + d;
+            const uint64_t at = (uint64_t(out_row) * a.query_heads + kv_head * groups + h) * kDim + d;
             const float inverse = 1.0f / lsum;
             const float merged = sum + 0.0f;
             if constexpr (QF == LK_BF16) reinterpret_cast<uint16_t*>(a.out)[at] = to_bf16(merged * inverse);
             else reinterpret_cast<float*>(a.out)[at] = merged * inverse;
             continue;
         }
-        const uint64_t slot = (uint64_t(seq) * a.query_heads + kv_head * groups + h) * a.splits + split;
+        const uint64_t slot = (uint64_t(out_row) * a.query_heads + kv_head * groups + h) * a.splits + split;
         a.partial_acc[slot * kDim + d] = sum;
         if (d == 0) {
             a.partial_ml[2 * slot] = best;
@@ -866,7 +872,8 @@ __device__ __forceinline__ void combine_dim128(const DecodeArgs& a, void* out, u
     const uint32_t lane = threadIdx.x;
     const uint32_t quad = lane % 32, half = lane / 32;
     const int32_t length = a.lengths[uint64_t(seq) * a.lengths_stride];
-    const uint64_t base = (uint64_t(seq) * a.query_heads + qh) * a.splits;
+    const uint64_t out_row = uint64_t(blockIdx.y * a.batch + seq) * a.query_heads + qh;  // (layer, sequence, head)
+    const uint64_t base = out_row * a.splits;
     const float* ml = a.partial_ml + 2 * base;
     const f32x4* acc = reinterpret_cast<const f32x4*>(a.partial_acc + base * kDim);
     // Lane l holds the (m, l) of splits l and 64 + l.
@@ -924,7 +931,7 @@ __device__ __forceinline__ void combine_dim128(const DecodeArgs& a, void* out, u
     for (int i = 0; i < 4; ++i) sum[i] += __shfl_xor(sum[i], 32, kWave);
     if (half != 0) return;
     const float inverse = 1.0f / total;
-    const uint64_t at = (uint64_t(seq) * a.query_heads + qh) * kDim + 4 * quad;
+    const uint64_t at = out_row * kDim + 4 * quad;
     if constexpr (QF == LK_BF16) {
         const uint32_t lo = uint32_t(to_bf16(sum[0] * inverse)) | (uint32_t(to_bf16(sum[1] * inverse)) << 16);
         const uint32_t hi = uint32_t(to_bf16(sum[2] * inverse)) | (uint32_t(to_bf16(sum[3] * inverse)) << 16);
@@ -952,7 +959,8 @@ __global__ __launch_bounds__(kWave) void decode_combine_quarter(DecodeArgs a, vo
     const uint32_t quarter = blockIdx.x % 4, pair = blockIdx.x / 4;
     const uint32_t seq = pair / a.query_heads, qh = pair % a.query_heads;
     const int32_t length = a.lengths[uint64_t(seq) * a.lengths_stride];
-    const uint64_t base = (uint64_t(seq) * a.query_heads + qh) * a.splits;
+    const uint64_t out_row = uint64_t(blockIdx.y * a.batch + seq) * a.query_heads + qh;  // (layer, sequence, head)
+    const uint64_t base = out_row * a.splits;
     const float* ml = a.partial_ml + 2 * base;
     const f32x4* acc = reinterpret_cast<const f32x4*>(a.partial_acc + base * kDim) + quarter * 8 + col;
     float lane_m[kPages], lane_l[kPages];
@@ -1000,7 +1008,7 @@ __global__ __launch_bounds__(kWave) void decode_combine_quarter(DecodeArgs a, vo
         for (int i = 0; i < 4; ++i) sum[i] += __shfl_xor(sum[i], mask, kWave);
     if (grp != 0) return;
     const float inverse = 1.0f / total;
-    const uint64_t at = (uint64_t(seq) * a.query_heads + qh) * kDim + 32 * quarter + 4 * col;
+    const uint64_t at = out_row * kDim + 32 * quarter + 4 * col;
     if constexpr (QF == LK_BF16) {
         const uint32_t lo = uint32_t(to_bf16(sum[0] * inverse)) | (uint32_t(to_bf16(sum[1] * inverse)) << 16);
         const uint32_t hi = uint32_t(to_bf16(sum[2] * inverse)) | (uint32_t(to_bf16(sum[3] * inverse)) << 16);
@@ -1024,7 +1032,8 @@ __global__ __launch_bounds__(kWave) void decode_combine(DecodeArgs a, void* out)
     const uint32_t qh = blockIdx.x % a.query_heads;
     const uint32_t seq = blockIdx.x / a.query_heads;
     const int32_t length = a.lengths[uint64_t(seq) * a.lengths_stride];
-    const uint64_t base = (uint64_t(seq) * a.query_heads + qh) * a.splits;
+    const uint64_t out_row = uint64_t(blockIdx.y * a.batch + seq) * a.query_heads + qh;  // (layer, sequence, head)
+    const uint64_t base = out_row * a.splits;
     const float* ml = a.partial_ml + 2 * base;
     const float* acc = a.partial_acc + base * a.head_dim;
     constexpr uint32_t kPer = kMaxGenericDim / kWave;
@@ -1092,7 +1101,7 @@ __global__ __launch_bounds__(kWave) void decode_combine(DecodeArgs a, void* out)
         const uint32_t d = lane + i * kWave;
         if (d >= a.head_dim) continue;
         const float value = sum[i] * inverse;
-        const uint64_t at = (uint64_t(seq) * a.query_heads + qh) * a.head_dim + d;
+        const uint64_t at = out_row * a.head_dim + d;
         if constexpr (QF == LK_BF16) reinterpret_cast<uint16_t*>(out)[at] = to_bf16(value);
         else reinterpret_cast<float*>(out)[at] = value;
     }

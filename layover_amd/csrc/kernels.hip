@@ -165,13 +165,17 @@ bool tiled_decode(const lk_decode_shape& s, const void* q, const void* pool) {
     return s.head_dim % 8 == 0 && s.head_dim <= kMaxGenericDim && aligned(q, 4) && aligned(pool, 4);
 }
 
+// Layers a launch covers, and the rows between two layers' queries (LK_DECODE_LAYERS).
+uint32_t layer_count(const lk_decode_shape& s) { return std::max((s.flags >> 8) & 0xFFu, 1u); }
+uint32_t layer_rows(const lk_decode_shape& s) { return s.flags >> 16; }
+
 // Whether a shape belongs to the tiled kernel; misaligned pools of other shapes use its plan too.
 bool tiled_shape(const lk_decode_shape& s) {
     return !(s.slots == kSlots && s.head_dim == kDim && s.kv_format != LK_F32 && s.query_heads / s.kv_heads <= kMaxHeads);
 }
 
 uint64_t partial_bytes(const lk_decode_shape& s, uint64_t splits) {
-    return uint64_t(s.batch) * s.query_heads * splits * (uint64_t(s.head_dim) + 2) * sizeof(float);
+    return uint64_t(s.batch) * layer_count(s) * s.query_heads * splits * (uint64_t(s.head_dim) + 2) * sizeof(float);
 }
 
 // Plan of the tiled kernel, in tiles of 16 tokens of one KV head (and 16 query heads): 8 waves a
@@ -214,7 +218,7 @@ Geometry geometry(const lk_decode_shape& s, const void* pool = nullptr) {
     g.fast = pool != nullptr && fast_decode(s, pool);
     // Work units counted per KV head for both kernels, so the split count (and with it the
     // workspace size) does not depend on which kernel runs.
-    const uint64_t units = uint64_t(s.batch) * s.kv_heads;
+    const uint64_t units = uint64_t(s.batch) * layer_count(s) * s.kv_heads;
     // At most 256 blocks per split: the fast kernel's waves hold their block ids one per lane.
     //
     // Blocks per split, a power of two in [8, 256]. Large batches aim at about 4,096
@@ -258,12 +262,26 @@ void check_shape(const lk_decode_shape& s) {
     require(s.kv_format == LK_BF16 || s.kv_format == LK_F32 || s.kv_format == LK_FP8_RECORD, "unknown KV format");
     require(s.head_dim <= kMaxGenericDim || (s.slots == kSlots && s.head_dim == kDim), "head_dim above 256 is not supported");
     require(s.slots <= 1024, "more than 1024 slots per block is not supported");
-    require((s.flags & ~uint32_t(LK_DECODE_SHARED_BLOCKS)) == 0, "unknown decode flags");
+    require((s.flags & 0xFFu & ~uint32_t(LK_DECODE_SHARED_BLOCKS)) == 0, "unknown decode flags");
+    require((s.flags >> 8) == 0 || (layer_count(s) <= s.layers - s.layer && layer_rows(s) >= s.batch && (s.flags & 0xFF00u) != 0),
+            "the layers of a decode launch must exist and hold their rows");
 }
 
-// Workspace: split partials, acc [batch, query_heads, splits, head_dim] then (m, l) pairs.
+// The shape of one layer of a launch of several.
+lk_decode_shape one_layer(const lk_decode_shape& s, uint32_t at) {
+    lk_decode_shape one = s;
+    one.layer += at;
+    one.flags &= 0xFFu;
+    return one;
+}
+
+// Workspace: split partials, acc [layers, batch, query_heads, splits, head_dim] then (m, l) pairs. Several
+// layers run as one launch, or (shapes and pools the matrix-core kernel does not take) one after
+// the other in the same space.
 uint64_t workspace_bytes(const lk_decode_shape& s) {
-    return partial_bytes(s, geometry(s).splits);
+    const uint64_t bytes = partial_bytes(s, geometry(s).splits);
+    if (layer_count(s) == 1) return bytes;
+    return std::max(bytes, workspace_bytes(one_layer(s, 0)));
 }
 
 // Waves per workgroup of the matrix-core kernel: 4 when the grid gives the CUs two or more
@@ -273,19 +291,22 @@ uint64_t workspace_bytes(const lk_decode_shape& s) {
 uint32_t decode_waves(const DecodeArgs& a, uint64_t grid) {
     const uint32_t forced = env_waves();
     if (forced == 4 || (forced == 8 && a.groups <= 8)) return forced;
+    // Several layers of short tables: 8 waves write the outputs of a row's only split themselves.
+    if (a.layer_count > 1 && a.splits == 1 && a.groups <= 8) return 8;
     if (grid >= 2ull * compute_units()) return 4;
     return a.groups <= 8 ? 8 : 4;
 }
 
 template <int KV, int QF, bool kAppend>
-void launch_split_mfma_as(const DecodeArgs& a, uint32_t waves, uint32_t grid, hipStream_t stream) {
-    const dim3 block(kWave * waves);
+void launch_split_mfma_as(const DecodeArgs& a, uint32_t workgroups, hipStream_t stream) {
+    const uint32_t waves = a.waves;
+    const dim3 block(kWave * waves), grid(workgroups, a.layer_count);
     if (a.shared_blocks) {
-        if (waves == 8) hipLaunchKernelGGL((decode_split_mfma<KV, QF, 8, false, kAppend>), dim3(grid), block, 0, stream, a);
-        else hipLaunchKernelGGL((decode_split_mfma<KV, QF, 4, false, kAppend>), dim3(grid), block, 0, stream, a);
+        if (waves == 8) hipLaunchKernelGGL((decode_split_mfma<KV, QF, 8, false, kAppend>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((decode_split_mfma<KV, QF, 4, false, kAppend>), grid, block, 0, stream, a);
     } else {
-        if (waves == 8) hipLaunchKernelGGL((decode_split_mfma<KV, QF, 8, true, kAppend>), dim3(grid), block, 0, stream, a);
-        else hipLaunchKernelGGL((decode_split_mfma<KV, QF, 4, true, kAppend>), dim3(grid), block, 0, stream, a);
+        if (waves == 8) hipLaunchKernelGGL((decode_split_mfma<KV, QF, 8, true, kAppend>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((decode_split_mfma<KV, QF, 4, true, kAppend>), grid, block, 0, stream, a);
     }
 }
 
@@ -293,9 +314,8 @@ void launch_split_mfma_as(const DecodeArgs& a, uint32_t waves, uint32_t grid, hi
 // plain decode does not reserve the write's registers.
 template <int KV, int QF>
 void launch_split_mfma(const DecodeArgs& a, uint32_t grid, hipStream_t stream) {
-    const uint32_t waves = decode_waves(a, grid);
-    if (a.write_block != nullptr) launch_split_mfma_as<KV, QF, true>(a, waves, grid, stream);
-    else launch_split_mfma_as<KV, QF, false>(a, waves, grid, stream);
+    if (a.write_block != nullptr) launch_split_mfma_as<KV, QF, true>(a, grid, stream);
+    else launch_split_mfma_as<KV, QF, false>(a, grid, stream);
 }
 
 // Above this many splits the merge runs as four workgroups per (sequence, query head), one per
@@ -321,10 +341,10 @@ void launch_decode(const DecodeArgs& a, const Geometry& g, int kv, void* out, hi
         else hipLaunchKernelGGL((decode_split_generic<LK_FP8_RECORD, QF>), dim3(uint32_t(grid)), dim3(kWave), 0, stream, a);
     }
     if (a.out != nullptr) return;  // the split kernel wrote the output
-    const dim3 grid(a.batch * a.query_heads);
+    const dim3 grid(a.batch * a.query_heads, a.layer_count);
     if (!vector_combine_fits(a)) hipLaunchKernelGGL((decode_combine<QF>), grid, dim3(kWave), 0, stream, a, out);
     else if (a.splits > kQuarterSplits) {
-        const dim3 quarters(a.batch * a.query_heads * 4);
+        const dim3 quarters(a.batch * a.query_heads * 4, a.layer_count);
         if (a.splits <= kWave) hipLaunchKernelGGL((decode_combine_quarter<QF, false>), quarters, dim3(kWave), 0, stream, a, out);
         else hipLaunchKernelGGL((decode_combine_quarter<QF, true>), quarters, dim3(kWave), 0, stream, a, out);
     } else if (a.splits <= kWave) hipLaunchKernelGGL((decode_combine_vector<QF, false>), grid, dim3(kWave), 0, stream, a, out);
@@ -642,6 +662,22 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     require(q && pool && table && lengths && out && workspace, "null q, pool, table, lengths, out or workspace");
     require(workspace_bytes >= ::lk::workspace_bytes(s), "workspace smaller than lk_paged_decode_workspace");
     require(aligned(workspace, 4), "workspace must be 4-byte aligned");
+    if (layer_count(s) > 1 && !fast_decode(s, pool)) {
+        const uint64_t row_elems = uint64_t(s.query_heads) * s.head_dim, token_elems = uint64_t(s.kv_heads) * s.head_dim;
+        const uint64_t elem = s.q_format == LK_BF16 ? 2 : 4;
+        for (uint32_t i = 0; i < layer_count(s); ++i) {
+            TokenWrite layer_write{};
+            if (write != nullptr) {
+                layer_write = *write;
+                layer_write.k = static_cast<const uint16_t*>(write->k) + i * layer_rows(s) * token_elems;
+                layer_write.v = static_cast<const uint16_t*>(write->v) + i * layer_rows(s) * token_elems;
+            }
+            run_decode(one_layer(s, i), static_cast<const uint8_t*>(q) + i * layer_rows(s) * row_elems * elem, pool, table, lengths,
+                       static_cast<uint8_t*>(out) + uint64_t(i) * s.batch * row_elems * elem, workspace, workspace_bytes,
+                       write != nullptr ? &layer_write : nullptr, st);
+        }
+        return;
+    }
     Geometry g = geometry(s, pool);
     g.tiled = !g.fast && tiled_decode(s, q, pool) ? tiled_plan(s).waves : 0;
     DecodeArgs a{};
@@ -650,7 +686,7 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     a.table = table;
     a.lengths = lengths;
     a.partial_acc = static_cast<float*>(workspace);
-    a.partial_ml = a.partial_acc + uint64_t(s.batch) * s.query_heads * g.splits * s.head_dim;
+    a.partial_ml = a.partial_acc + uint64_t(s.batch) * layer_count(s) * s.query_heads * g.splits * s.head_dim;
     a.batch = s.batch;
     a.query_heads = s.query_heads;
     a.kv_heads = s.kv_heads;
@@ -665,6 +701,9 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     a.groups = s.query_heads / s.kv_heads;
     a.splits = g.splits;
     a.bps = g.bps;
+    a.layer_count = layer_count(s);
+    a.layer_rows = layer_rows(s);
+    a.waves = decode_waves(a, uint64_t(s.batch) * a.layer_count * g.splits * s.kv_heads);
     a.order = env_order();
     a.shared_blocks = (s.flags & LK_DECODE_SHARED_BLOCKS) != 0;
     a.vector_combine = aligned(workspace, 16) && aligned(out, s.q_format == LK_BF16 ? 8 : 16);
@@ -675,7 +714,7 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     // workgroups: the split kernel writes the output. (The 4-wave kernel has no such branch,
     // which measurably costs the large-batch loop.) LAYOVER_DECODE_COMBINE keeps the combine
     // launch (for comparisons).
-    if (g.fast && g.splits == 1 && env_combine() == 0 && decode_waves(a, uint64_t(s.batch) * s.kv_heads) == 8) a.out = out;
+    if (g.fast && g.splits == 1 && env_combine() == 0 && a.waves == 8) a.out = out;
     if (g.tiled && g.splits == 1 && env_combine() == 0) a.out = out;
     require(aligned(pool, s.kv_format == LK_F32 ? 4 : (s.kv_format == LK_BF16 ? 2 : 1)), "misaligned pool");
     if (write != nullptr) {
@@ -791,6 +830,7 @@ LK_EXPORT int lk_paged_decode_static(const lk_decode_shape* shape, const void* q
     return lk::guarded([&] {
         lk::require(shape != nullptr, "null shape");
         lk::check_shape(*shape);
+        lk::require(lk::layer_count(*shape) == 1, "lk_paged_decode_static takes one layer");
         const uint64_t need = lk::workspace_bytes(*shape);
         if (need > lk::kStaticScratchBytes)
             throw lk::Invalid("lk_paged_decode_static: this shape needs " + std::to_string(need) + " bytes of split partials, above the " +

@@ -185,12 +185,14 @@ def validate(q, pool, layer, block_table, lengths, kv_groups) -> int:
     return listed
 
 
-def decode_shape(q, pool, layer, block_table, kv_groups, lengths=None, shared_blocks: bool = False) -> _lib.DecodeShape:
+def decode_shape(q, pool, layer, block_table, kv_groups, lengths=None, shared_blocks: bool = False, layer_count: int = 1,
+                 layer_rows: int = 0) -> _lib.DecodeShape:
     """The launch's shape; the table's row stride and the lengths' stride are taken from the
     tensors, so columns of a packed row block (PagedKVCache.decode_rows) pass without a copy,
     as the reference's launcher passes strides (triton_decode.py:131-179). shared_blocks sets
     LK_DECODE_SHARED_BLOCKS: rows read some of the same blocks, so the kernel keeps tiles in
-    the caches instead of streaming them (the same results, a different speed)."""
+    the caches instead of streaming them (the same results, a different speed). layer_count above
+    1 sets LK_DECODE_LAYERS: that many layers from `layer` on in one launch, layer_rows rows apart."""
     batch, query_heads, head_dim = q.shape
     _, _, layers, kv_heads, slots, _ = pool.shape
     kv_format = _lib.LK_FP8_RECORD if _is_fp8(pool) else _FORMATS[pool.dtype]
@@ -198,7 +200,8 @@ def decode_shape(q, pool, layer, block_table, kv_groups, lengths=None, shared_bl
     lengths_stride = lengths.stride(0) if lengths is not None and lengths.dim() == 1 else 1
     return _lib.DecodeShape(batch, query_heads, kv_heads, head_dim, layers, slots, layer, block_table.shape[1],
                             _FORMATS[q.dtype], kv_format, 1.0 / math.sqrt(head_dim), table_stride, lengths_stride,
-                            _lib.LK_DECODE_SHARED_BLOCKS if shared_blocks else 0)
+                            (_lib.LK_DECODE_SHARED_BLOCKS if shared_blocks else 0)
+                            | (layer_count << 8 | layer_rows << 16 if layer_count > 1 else 0))
 
 
 def _check_layout(q, block_table, lengths, out) -> None:
@@ -259,6 +262,44 @@ def run_kernel_append(q, pool, layer, block_table, lengths, kv_groups, write_blo
         raise ValueError("one written token per decode row")
     lib = _lib.load()
     shape = decode_shape(q, pool, layer, block_table, kv_groups, lengths, shared_blocks)
+    need = int(lib.lk_paged_decode_workspace(shape))
+    if workspace is None or workspace.numel() < need:
+        workspace = torch.empty(max(need, 4), dtype=torch.uint8, device=q.device)
+    _lib.check(
+        lib.lk_paged_decode_append(shape, q.data_ptr(), storage.data_ptr(), block_table.data_ptr(), lengths.data_ptr(),
+                                   write_blocks.data_ptr(), write_slots.data_ptr(), write_blocks.stride(0), k.data_ptr(), v.data_ptr(),
+                                   out.data_ptr(), workspace.data_ptr(), workspace.numel(), _lib.current_stream(q.device))
+    )
+
+
+def run_kernel_append_layers(q, pool, layer, block_table, lengths, kv_groups, write_blocks, write_slots, k, v, out, workspace=None,
+                             shared_blocks: bool = False) -> None:
+    """run_kernel_append of q.shape[0] layers from `layer` on, for callers that hold every layer's
+    queries at once: q [layers, batch, query_heads, head_dim], k and v [layers, batch, kv_heads,
+    head_dim], with any number of rows between two layers (the same for all three), out contiguous
+    in q's shape. Up to 255 layers and 65,535 rows between them; one launch where the shape allows."""
+    count, batch = q.shape[0], q.shape[1]
+    if out.shape != q.shape or not out.is_contiguous() or k.shape[0] != count or v.shape[0] != count:
+        raise ValueError("q, k, v and out must hold the same layers, out contiguous")
+    rows = q.stride(0) // (q.shape[2] * q.shape[3]) if count > 1 else batch
+    for name, t in (("q", q), ("k", k), ("v", v)):
+        if count > 1 and t.stride(0) != rows * t.shape[2] * t.shape[3]:
+            raise ValueError(f"{name} must have whole rows between its layers, as many as the others")
+    if not 1 <= count <= 255 or not batch <= rows < 65536:
+        raise ValueError(f"{count} layers of {rows} rows for a batch of {batch} are not one launch's")
+    _check_layout(q[0], block_table, lengths, out[0])
+    if _is_fp8(pool):
+        storage, layers, kv_heads, head_dim = pool.records, pool.layers, pool.kv_heads, pool.head_dim
+    else:
+        if pool.dtype != torch.bfloat16:
+            raise ValueError("a fused write needs a BF16 or FP8-record pool")
+        storage, layers, kv_heads, head_dim = pool, pool.shape[2], pool.shape[3], pool.shape[5]
+    if layer + count > layers:
+        raise ValueError(f"layers {layer} to {layer + count - 1} are not all among {layers}")
+    if _check_token_write(storage.device, layers, kv_heads, head_dim, write_blocks, write_slots, layer, k[0], v[0]) != batch:
+        raise ValueError("one written token per decode row")
+    lib = _lib.load()
+    shape = decode_shape(q[0], pool, layer, block_table, kv_groups, lengths, shared_blocks, count, rows)
     need = int(lib.lk_paged_decode_workspace(shape))
     if workspace is None or workspace.numel() < need:
         workspace = torch.empty(max(need, 4), dtype=torch.uint8, device=q.device)
