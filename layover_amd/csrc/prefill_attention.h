@@ -666,48 +666,46 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
                 if (int32_t(key0 + b * kSlots + 4 * g + r) > limit[set]) s[b][r] = -INFINITY;
     };
 
-    // Rescaling. The state of a row is rescaled only when a score exceeds its running maximum
-    // by more than kRescaleThreshold (log2 units), which is rare after the first steps. The
-    // common path therefore only compares each lane's own maximum with a precomputed limit:
-    // for BF16 pools on the raw scores against (m + threshold) / scale, for FP8 pools on the
-    // scaled scores of each block. Only when some lane exceeds it are the row maxima reduced
-    // over the lane groups (row n lives in lanes n, n + 16, n + 32, n + 48) and the state
-    // rescaled. A lane that misses the limit by rounding at most lets a weight reach 2^8 times
-    // an ulp more, which the threshold exists to bound anyway.
-    float raw_limit[2] = {-INFINITY, -INFINITY};  // BF16: (m + threshold) / scale per set
-    auto lane_max = [&](const f32x4 (&s)[2], const Factors& f) __attribute__((always_inline)) {
-        if constexpr (KV == LK_BF16) {
-            return fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-        } else {
-            float top_b[2];
+    // Rescaling. The state of a row is rescaled only when a score exceeds its running maximum by more
+    // than kRescaleThreshold (log2 units), rare after the first steps; weights then stay below 2^8,
+    // which the threshold exists to bound.
+    // BF16 pools keep in m the maximum plus kRescaleThreshold - 1, so that the weights in use are
+    // below 2 exactly while no score exceeds the threshold, and find that out from the weights
+    // themselves: a BF16 of 2 or more (infinity and NaN too) has its top exponent bit set, so one OR over
+    // a lane's packed weights and one compare stand for the maxima of its scores. `raise` then takes
+    // the row's maximum over the lane groups (row n lives in lanes n, n + 16, n + 32 and n + 48).
+    // FP8 pools compare each lane's own maximum of the scaled scores first.
+    constexpr float kHeadroom = kRescaleThreshold - 1.0f;
+    auto rescale_state = [&](int set, float next) __attribute__((always_inline)) {
+        const float alpha = merge_weight(m[set], next);
+        m[set] = next;
+        l[set] *= alpha;
 #pragma unroll
-            for (int b = 0; b < 2; ++b) top_b[b] = fmaxf(fmaxf(fmaxf(s[b][0], s[b][1]), s[b][2]), s[b][3]) * f.k[b];
-            return fmaxf(top_b[0], top_b[1]);
+        for (int r = 0; r < 4; ++r) {
+            const float factor = __shfl(alpha, int(4 * g + r), kWave);
+            sums[set][r] *= factor;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[set][e][r] *= factor;
         }
     };
-    auto exceeds = [&](int set, float lane_top) __attribute__((always_inline)) {
-        if constexpr (KV == LK_BF16) return lane_top > raw_limit[set];
-        else return lane_top > m[set] + kRescaleThreshold;
+    auto raise = [&](int set, const f32x4 (&s)[2]) __attribute__((always_inline)) {
+        float top = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+        top = max_over_lane_groups(top) * a.scale_log2 + kHeadroom;
+        rescale_state(set, top > m[set] + 1.0f ? top : m[set]);
+    };
+    auto lane_max = [&](const f32x4 (&s)[2], const Factors& f) __attribute__((always_inline)) {
+        float top_b[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) top_b[b] = fmaxf(fmaxf(fmaxf(s[b][0], s[b][1]), s[b][2]), s[b][3]) * f.k[b];
+        return fmaxf(top_b[0], top_b[1]);
     };
     auto rescale = [&](const float (&lane_top)[2]) __attribute__((always_inline)) {
-        if (__builtin_expect(__any(exceeds(0, lane_top[0]) || exceeds(1, lane_top[1])), 0)) {
+        if (__builtin_expect(__any(lane_top[0] > m[0] + kRescaleThreshold || lane_top[1] > m[1] + kRescaleThreshold), 0)) {
             asm volatile("" ::: "memory");
 #pragma unroll
             for (int set = 0; set < 2; ++set) {
-                float top = max_over_lane_groups(lane_top[set]);
-                if constexpr (KV == LK_BF16) top *= a.scale_log2;
-                const float next = top > m[set] + kRescaleThreshold ? top : m[set];
-                const float alpha = merge_weight(m[set], next);
-                m[set] = next;
-                if constexpr (KV == LK_BF16) raw_limit[set] = (next + kRescaleThreshold) / a.scale_log2;
-                l[set] *= alpha;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float factor = __shfl(alpha, int(4 * g + r), kWave);
-                    sums[set][r] *= factor;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) o[set][e][r] *= factor;
-                }
+                const float top = max_over_lane_groups(lane_top[set]);
+                rescale_state(set, top > m[set] + kRescaleThreshold ? top : m[set]);
             }
         }
     };
@@ -740,12 +738,18 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
     };
 
     PrefillStaged staged;
-    // One step, per set: scores, mask and maximum, then (after a rare rescale of both sets)
-    // weights and PV, in two straight stretches that the scheduler fills from both sets. Then
-    // the next step's tiles go into the other buffer and the one after into registers. Steps
-    // that need the causal mask (and the chunk-end V mask, which only the last step can need)
-    // run in a second copy of the loop. Forcing an MFMA/VALU interleave with scheduling
-    // barriers measured 4% slower: the two waves on each SIMD already overlap each other.
+    // One step: set 0's scores, then set 1's beside set 0's exponentials, set 0's PV beside set 1's
+    // exponentials, set 1's PV: the wave's VALU work always has independent MFMAs beside it. The
+    // scheduling barrier after set 0's scores keeps the two sets' QK products from being mixed, which
+    // would leave set 0's softmax nothing to run beside. Then the next step's tiles go into the other
+    // buffer and the one after into registers. Steps that need the causal mask (and the chunk-end V
+    // mask, which only the last step can need) run in a second copy of the loop.
+    // Measured on MI355X (A/B on one box, 2,048 tokens ending a 32,768 context, 2,048 at 0, and 509 at
+    // 8,203 of an FP8 pool): 951, 42.2 and 90.0 us per layer with the maxima of both sets ahead of any
+    // exponential; 926, 41.3 and 88.0 with the check on the weights; 877, 40.8 and 84.9 with the sets
+    // staggered. On top of that: MFMAs and VALU work dealt one to 2, 3 or 4 by scheduling groups 959,
+    // 943 and 959 against 940 us on another box; K of the next step read ahead of set 1's PV 934 us
+    // against 877 (its registers spill the loop's).
     auto run_step = [&](uint32_t step, auto masked_tag) __attribute__((always_inline)) {
         constexpr bool kMasked = decltype(masked_tag)::value;
         if constexpr (KV == LK_BF16) {
@@ -763,20 +767,16 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
         values(step, vb);
         f32x4 s[2][2];
         scores(0, kk, s[0]);
-        scores(1, kk, s[1]);
-        if constexpr (kMasked) mask(step, 0, s[0]);
-        float top[2];
-        // The softmax stretch (row maxima, rescale, exponentials, with set 0's PV in between)
-        // runs at raised wave priority: the SIMD's other wave is then mostly in its matrix-core
-        // stretch, whose MFMAs keep running while this wave's dependent VALU chain is issued
-        // first. Measured on MI355X (2,048 tokens ending a 32,768 context): 1.094 -> 1.023 ms
-        // per layer; raising it for the QK MFMAs instead, or dropping it around set 0's PV, was
-        // 1.08-1.11 and 1.07 ms. With the steps paired it still gains 1-2% there (1.059-1.067
-        // against 1.079-1.081 ms on one box), and under the max-ilp scheduling the prefill kernels
-        // build with (0.991-1.001 against 1.003-1.010 ms).
+        __builtin_amdgcn_sched_barrier(0);
+        // Raised wave priority from here to set 1's PV: the SIMD's other wave is then mostly in a
+        // matrix-core stretch, whose MFMAs keep running while this wave's dependent chain is issued
+        // first. From set 0's scores on 985 us per layer on the long chunk, from here 940, after set
+        // 1's scores 1,001, never 1,025 (same box; the priority instruction also keeps what stands
+        // before it from being scheduled past it).
         __builtin_amdgcn_s_setprio(1);
-        top[0] = lane_max(s[0], f);
+        scores(1, kk, s[1]);
         if constexpr (kMasked) {
+            mask(step, 0, s[0]);
             mask(step, 1, s[1]);
             // Keys at or past the chunk's end hold anything: zero their V (0 * NaN is NaN).
             const uint32_t key0 = step * 2 * kSlots;
@@ -795,13 +795,29 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
                 }
             }
         }
-        top[1] = lane_max(s[1], f);
-        rescale(top);
-        const bf16x8 p0 = weights(0, s[0], f);
-        accumulate(0, p0, vb);
-        const bf16x8 p1 = weights(1, s[1], f);
-        __builtin_amdgcn_s_setprio(0);
-        accumulate(1, p1, vb);
+        if constexpr (KV == LK_BF16) {
+#pragma unroll
+            for (int set = 0; set < 2; ++set) {
+                bf16x8 p = weights(set, s[set], f);
+                const u32x4 bits = __builtin_bit_cast(u32x4, p);
+                if (__builtin_expect(__any(((bits[0] | bits[1] | bits[2] | bits[3]) & 0x40004000u) != 0), 0)) {
+                    asm volatile("" ::: "memory");
+                    raise(set, s[set]);
+                    p = weights(set, s[set], f);
+                }
+                if (set == 1) __builtin_amdgcn_s_setprio(0);
+                accumulate(set, p, vb);
+            }
+        } else {
+            __builtin_amdgcn_s_setprio(1);
+            const float top[2] = {lane_max(s[0], f), lane_max(s[1], f)};
+            rescale(top);
+            const bf16x8 p0 = weights(0, s[0], f);
+            accumulate(0, p0, vb);
+            const bf16x8 p1 = weights(1, s[1], f);
+            __builtin_amdgcn_s_setprio(0);
+            accumulate(1, p1, vb);
+        }
         if constexpr (KV == LK_BF16) {
             if ((step - first_step) % 2 == 1 || step + 1 == steps) step_barrier();
         } else {
