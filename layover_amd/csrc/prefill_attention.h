@@ -592,7 +592,9 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[set][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    const bf16x8 ones = as_bf16x8(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
+    u32x4 one_bits = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+    if constexpr (KV == LK_BF16) asm volatile("" : "+v"(one_bits));  // held, not moved together again in every step
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, one_bits);
 
     // Transposing V reads: lane 4t + q of group g fetches key 4g + t, dims 16e + 4q .. +3,
     // i.e. bytes 8q .. 8q+7 of chunks 2e, 2e + 1 (region e / 2, offset 32 (e % 2)).
@@ -749,7 +751,8 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
     // exponential; 926, 41.3 and 88.0 with the check on the weights; 877, 40.8 and 84.9 with the sets
     // staggered. On top of that: MFMAs and VALU work dealt one to 2, 3 or 4 by scheduling groups 959,
     // 943 and 959 against 940 us on another box; K of the next step read ahead of set 1's PV 934 us
-    // against 877 (its registers spill the loop's).
+    // against 877 (its registers spill the loop's); the weight sums by dot products of the packed pairs
+    // instead of the MFMA against ones 922 against 875: VALU slots are as scarce as matrix ones.
     auto run_step = [&](uint32_t step, auto masked_tag) __attribute__((always_inline)) {
         constexpr bool kMasked = decltype(masked_tag)::value;
         if constexpr (KV == LK_BF16) {
@@ -768,11 +771,12 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
         f32x4 s[2][2];
         scores(0, kk, s[0]);
         __builtin_amdgcn_sched_barrier(0);
-        // Raised wave priority from here to set 1's PV: the SIMD's other wave is then mostly in a
+        // Raised wave priority from here to the end of set 1's PV: the SIMD's other wave is then mostly in a
         // matrix-core stretch, whose MFMAs keep running while this wave's dependent chain is issued
         // first. From set 0's scores on 985 us per layer on the long chunk, from here 940, after set
         // 1's scores 1,001, never 1,025 (same box; the priority instruction also keeps what stands
-        // before it from being scheduled past it).
+        // before it from being scheduled past it); lowered before set 1's PV 868 against 865 there, 84.2
+        // against 82.9 us on the 509-token chunk.
         __builtin_amdgcn_s_setprio(1);
         scores(1, kk, s[1]);
         if constexpr (kMasked) {
@@ -805,8 +809,8 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
                     raise(set, s[set]);
                     p = weights(set, s[set], f);
                 }
-                if (set == 1) __builtin_amdgcn_s_setprio(0);
                 accumulate(set, p, vb);
+                if (set == 1) __builtin_amdgcn_s_setprio(0);
             }
         } else {
             __builtin_amdgcn_s_setprio(1);
