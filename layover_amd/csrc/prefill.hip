@@ -7,6 +7,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <string>
@@ -21,10 +22,10 @@
 namespace lk {
 
 // Split-K plan for the LDS prefill kernel. Workgroups are (KV head, 128-row tile); a chunk
-// whose tiles do not give every CU two of them (short chunks against long histories) also
-// splits each tile's keys, at least 4 steps (128 keys) per split and at most kMaxKeySplits
-// splits, and merges the partials in prefill_merge. LAYOVER_PREFILL_SPLITS=n forces n
-// splits (tests), read per launch.
+// whose tiles do not give every CU two of them (short chunks against long histories) may also
+// split each tile's keys, at least 4 steps (128 keys) per split and at most kMaxKeySplits
+// splits, and merge the partials in prefill_merge: as many splits as split_cost finds cheapest.
+// LAYOVER_PREFILL_SPLITS=n forces n splits (tests), read per launch.
 //
 // FP8-record pools, given a workspace (lk_paged_prefill_split): the chunk's history is first
 // decoded, one layer, into a compact BF16 pool in the workspace (stage_history_2048: each
@@ -47,7 +48,9 @@ struct PrefillPlan {
 // prologue and epilogue); LAYOVER_PREFILL_PAIR_BIAS overrides it, read per launch. Measured on
 // MI355X, 2,048 tokens at position 0 (partner on the heavy remainder first): 0.049-0.051 ms per
 // layer at 8, 0.049 at 10, 0.050-0.051 at 12, 0.050-0.052 at 14-16 (two runs each, one box).
-constexpr int32_t kPairBias = 10;
+// The staggered step (prefill_attention.h) moved the optimum a little: 40.7, 40.5, 40.9 and 41.1 us at 6,
+// 8, 10 and 12.
+constexpr int32_t kPairBias = 8;
 
 // Key steps of a 128-row tile of the LDS kernel, and whether a CU pair divides its heavy
 // tile: the same arithmetic as prefill_mfma_lds's job plan.
@@ -66,6 +69,28 @@ bool any_pair_divides(const lk_prefill_shape& s, uint64_t row_tiles, int32_t bia
         if (cut < heavy_steps && uint64_t(heavy_steps - cut) * 8 >= heavy_steps) return true;
     }
     return false;
+}
+
+// Microseconds of a launch whose tiles run `splits` ways, from what the kernel measured on MI355X: a start
+// and an end of 6.5 us, 0.6 us a step for a workgroup alone on its CU, 0.78 for two that share one,
+// whole rounds of two per CU beyond that; and the merge, a launch (3 us) over partials written and read
+// at 5 TB/s. Model and measurement (8 KV heads x 4, us per layer): 391 tokens at 0 in 1, 2 and 3 splits
+// 14.3, 18.9, 22.6 and 14.3, 20.8, 23.7; 509 at 8,203 in 2 and 4 98, 76 and 96, 75; 1,000 at 1,000 in 1
+// and 2 44, 48 and 44, 47; 64 at 4,000 in 8 and 31 22, 26 and 23, 26. Splitting until every CU had two
+// workgroups, whatever the partials cost, took 23.7, 75, 47 and 26 us there, and 82 us for 1,900 tokens
+// at 300 (480 workgroups, short of 512) where one way takes 47.
+double split_cost(const lk_prefill_shape& s, uint32_t cus, uint64_t row_tiles, uint32_t steps, uint32_t splits) {
+    const uint64_t workgroups = row_tiles * s.kv_heads * splits, rounds = (workgroups + 2 * cus - 1) / (2 * cus);
+    const uint32_t groups = s.query_heads / s.kv_heads;
+    double each = (steps + splits - 1) / splits;
+    if (splits == 1 && workgroups > cus) {
+        // Heavy and light tiles share CUs (PrefillArgs::paired) and, where they differ, their steps.
+        const uint32_t light = lds_tile_steps(s.start, uint64_t(s.tokens) * groups, groups, 0);
+        each = std::min<double>(each, (steps + light + kPairBias) / 2.0 + 4.0);
+    }
+    double cost = 6.5 + each * (workgroups <= cus ? 0.6 : 0.78) * rounds;
+    if (splits > 1) cost += 3.0 + 2.0 * s.query_heads * double(s.tokens) * splits * (kDim + 2) * sizeof(float) / 5e6;
+    return cost;
 }
 
 PrefillPlan prefill_plan(const lk_prefill_shape& s) {
@@ -95,8 +120,17 @@ PrefillPlan prefill_plan(const lk_prefill_shape& s) {
     } else {
         const uint64_t workgroups = p.row_tiles * s.kv_heads, target = 2ull * compute_units();
         if (workgroups < target) {
-            const uint64_t fill = (target + workgroups - 1) / workgroups, cap = max_steps / 4;
-            wanted = uint32_t(fill < cap ? fill : cap);
+            const uint64_t fill = (target + workgroups - 1) / workgroups;
+            const uint32_t cap = uint32_t(std::min<uint64_t>({fill, max_steps / 4, kMaxKeySplits}));
+            wanted = 1;
+            double least = split_cost(s, uint32_t(target / 2), p.row_tiles, max_steps, 1);
+            for (uint32_t n = 2; n <= cap; ++n) {
+                const double cost = split_cost(s, uint32_t(target / 2), p.row_tiles, max_steps, n);
+                if (cost < least) {
+                    least = cost;
+                    wanted = n;
+                }
+            }
         }
     }
     const uint32_t most = kMaxKeySplits < max_steps ? kMaxKeySplits : max_steps;

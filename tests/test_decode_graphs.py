@@ -293,3 +293,17 @@ def test_plain_calls_are_told_from_those_the_checks_must_see(change, monkeypatch
         return
     expected = hip_decode.decode_shape(q, pool, layer, table, 2, lengths, True)
     assert [getattr(shape, name) for name, _ in shape._fields_] == [getattr(expected, name) for name, _ in expected._fields_]
+
+
+@pytest.mark.parametrize("tokens,start,splits", [(391, 0, 1), (1900, 300, 1), (1000, 1000, 1), (509, 8203, 4), (1024, 4096, 2)])
+def test_prefill_splits_only_where_the_partials_pay(tokens, start, splits, monkeypatch):
+    """The split plan weighs the steps a split saves against its partials: chunks that nearly fill the
+    GPU, or whose history is short, stay whole (their workspace is at most pair states), others split."""
+    from layover_amd.kernels import _lib
+
+    for name in ("LAYOVER_PREFILL_SPLITS", "LAYOVER_PREFILL_KERNEL", "LAYOVER_PREFILL_PAIR_BIAS"):
+        monkeypatch.delenv(name, raising=False)
+    monkeypatch.setenv("LAYOVER_PREFILL_PAIR_HALVES", "0")
+    shape = _lib.PrefillShape(tokens, start, 32, 8, 128, 36, 16, 3, _lib.LK_BF16, _lib.LK_BF16, 128**-0.5)
+    expected = 0 if splits == 1 else 32 * tokens * splits * 130 * 4
+    assert _lib.load().lk_paged_prefill_workspace(shape) == expected
