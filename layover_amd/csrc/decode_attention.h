@@ -283,8 +283,10 @@ __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(K
     uint32_t split, kv_head, seq;
     if (!decode_unit_of(a, blockIdx.x, &seq, &split, &kv_head)) return;
     const uint32_t groups = a.groups;
-    const uint32_t layer = a.layer + blockIdx.y;
-    const uint32_t in_row = blockIdx.y * a.layer_rows + seq, out_row = blockIdx.y * a.batch + seq;
+    // Only launches with the token write cover several layers.
+    const uint32_t layer_at = kAppend ? blockIdx.y : 0;
+    const uint32_t layer = a.layer + layer_at;
+    const uint32_t in_row = layer_at * a.layer_rows + seq, out_row = layer_at * a.batch + seq;
 
     // The split's block ids are loaded (one per lane, this wave's units) before the length
     // is known, bounded by the table width alone, so the two loads overlap; the length then

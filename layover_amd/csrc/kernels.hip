@@ -221,29 +221,45 @@ Geometry geometry(const lk_decode_shape& s, const void* pool = nullptr) {
     const uint64_t units = uint64_t(s.batch) * layer_count(s) * s.kv_heads;
     // At most 256 blocks per split: the fast kernel's waves hold their block ids one per lane.
     //
-    // Blocks per split, a power of two in [8, 256]. Large batches aim at about 4,096
-    // workgroups (at least 64 blocks each); FP8 records, whose tiles are half the bytes, at
-    // about 8,192: batch 32 at 1,024-32,768 tokens on distinct blocks 189.7 -> 186 us per layer,
-    // on shared blocks 153 -> 151.5 us, with 64 blocks a split instead of 128 (the same change
-    // slowed the BF16 decode, 288 -> 291.6 us on shared blocks). A grid that would leave CUs idle instead takes
-    // about one workgroup per CU: measured per layer at batch 1, 4,096 tokens 19.9 -> 12.8 us
-    // (BF16) with 16 splits instead of 4, and at 16,384 tokens 22.3 -> 20.3 us. An FP8-record
-    // table of at most 64 blocks stays one split, which writes the output itself with no merge
-    // launch (10.8 against 12.2 us at 1,024 tokens); BF16 tiles, twice the bytes, gain more from
-    // spreading (13.3 -> 11.8 us).
+    // Blocks per split, in [8, 256].
+    // Large batches: a power of two that aims at about 4,096 workgroups (at least 64 blocks each); FP8
+    // records, whose tiles are half the bytes, at about 8,192: batch 32 at 1,024-32,768 tokens on
+    // distinct blocks 189.7 -> 186 us per layer, on shared blocks 153 -> 151.5 us, with 64 blocks a
+    // split instead of 128 (the same change slowed the BF16 decode, 288 -> 291.6 us on shared blocks).
+    // Grids that would leave CUs idle: about one workgroup per CU and no more, since a CU holds one of
+    // 8 waves (measured per layer at batch 1, 4,096 tokens 19.9 -> 12.8 us BF16 with 16 splits instead
+    // of 4; batch 3 at 6,000 tokens 20.3 us in 6 splits of 64 blocks, 15.5 in 12 of 32).
+    // Short tables: one split, written by the split kernel itself with no merge launch, for
+    //   - FP8 records of at most 64 blocks (10.8 against 12.2 us at batch 1 and 1,024 tokens), and
+    //     BF16 of at most 16 (batch 1-16 at 200 tokens 8.3-10.2 -> 6.0-7.3 us);
+    //   - at most 112 blocks where the rows' KV heads give most CUs a workgroup, fewer for narrower
+    //     tables (BF16 at 700, 1,500 and 1,500 tokens, batch 16, 24 and 64: 14.3 -> 11.8, 35.0 -> 24.9,
+    //     65 -> 53.5 us; FP8 at 1,500, batch 24 and 64: 24.6 -> 15.6, 41.7 -> 32.4; batch 12 even). A
+    //     row that is much longer than the others is one workgroup's chain, so the line is not
+    //     drawn where even rows alone would have it (BF16 at 3,000, batch 32: 61 -> 53 us).
+    //   Rows of one launch's several layers stay split above 64 blocks (three rows of 600-2,000
+    //   tokens x 36 layers: 192 us a step in 64-block splits, 204 in one).
     uint32_t bps = env_bps() > 256 ? 256 : env_bps();
     if (bps == 0) {
-        const uint64_t work = units * s.table_width;
-        const uint64_t target = s.kv_format == LK_FP8_RECORD ? 8192 : 4096;
-        const uint64_t large = (work + target - 1) / target;
-        const uint64_t fill = (work + compute_units() - 1) / compute_units();
-        const uint64_t wanted = s.kv_format == LK_FP8_RECORD && s.table_width <= 64 ? 64 : std::max(large, std::min<uint64_t>(fill, 64));
-        bps = 8;
-        while (bps < wanted && bps < 256) bps *= 2;
+        const uint64_t work = units * s.table_width, width = s.table_width, cus = compute_units();
+        const bool fp8 = s.kv_format == LK_FP8_RECORD, writes = s.query_heads / s.kv_heads <= 8 && layer_count(s) == 1;
+        const uint64_t target = fp8 ? 8192 : 4096;
+        const uint64_t large = (work + target - 1) / target, fill = (work + cus - 1) / cus;
+        if (width <= (fp8 ? 64u : 16u) || (writes && width <= 112 && units >= std::min(2 * width, cus * 3 / 4))) {
+            bps = uint32_t(std::max<uint64_t>(width, 8));
+        } else if (fill < 64) {
+            const uint64_t splits = std::max<uint64_t>(cus / units, 1);
+            bps = uint32_t(std::max<uint64_t>((width + splits - 1) / splits, 8));
+        } else {
+            bps = 64;
+            while (bps < large && bps < 256) bps *= 2;
+        }
         if (tiled_shape(s)) {
-            // Partials that lk_paged_decode_static can hold, as long as the plan above keeps them so.
+            // Partials that lk_paged_decode_static can hold, as long as 64-block splits or larger keep them so.
             uint32_t tiled = tiled_plan(s).bps;
-            while (tiled < bps && partial_bytes(s, (s.table_width + tiled - 1) / tiled) > kStaticScratchBytes) ++tiled;
+            uint64_t most = 64;
+            while (most < large && most < 256) most *= 2;
+            while (tiled < most && partial_bytes(s, (s.table_width + tiled - 1) / tiled) > kStaticScratchBytes) ++tiled;
             bps = tiled;
         }
     }
@@ -276,8 +292,8 @@ lk_decode_shape one_layer(const lk_decode_shape& s, uint32_t at) {
 }
 
 // Workspace: split partials, acc [layers, batch, query_heads, splits, head_dim] then (m, l) pairs. Several
-// layers run as one launch, or (shapes and pools the matrix-core kernel does not take) one after
-// the other in the same space.
+// layers run as one launch, or (with no token write, or shapes and pools the matrix-core kernel does
+// not take) one after the other in the same space.
 uint64_t workspace_bytes(const lk_decode_shape& s) {
     const uint64_t bytes = partial_bytes(s, geometry(s).splits);
     if (layer_count(s) == 1) return bytes;
@@ -291,8 +307,8 @@ uint64_t workspace_bytes(const lk_decode_shape& s) {
 uint32_t decode_waves(const DecodeArgs& a, uint64_t grid) {
     const uint32_t forced = env_waves();
     if (forced == 4 || (forced == 8 && a.groups <= 8)) return forced;
-    // Several layers of short tables: 8 waves write the outputs of a row's only split themselves.
-    if (a.layer_count > 1 && a.splits == 1 && a.groups <= 8) return 8;
+    // Short tables: 8 waves write the outputs of a row's only split themselves.
+    if (a.splits == 1 && a.groups <= 8) return 8;
     if (grid >= 2ull * compute_units()) return 4;
     return a.groups <= 8 ? 8 : 4;
 }
@@ -662,7 +678,7 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     require(q && pool && table && lengths && out && workspace, "null q, pool, table, lengths, out or workspace");
     require(workspace_bytes >= ::lk::workspace_bytes(s), "workspace smaller than lk_paged_decode_workspace");
     require(aligned(workspace, 4), "workspace must be 4-byte aligned");
-    if (layer_count(s) > 1 && !fast_decode(s, pool)) {
+    if (layer_count(s) > 1 && (write == nullptr || !fast_decode(s, pool))) {
         const uint64_t row_elems = uint64_t(s.query_heads) * s.head_dim, token_elems = uint64_t(s.kv_heads) * s.head_dim;
         const uint64_t elem = s.q_format == LK_BF16 ? 2 : 4;
         for (uint32_t i = 0; i < layer_count(s); ++i) {

@@ -307,3 +307,15 @@ def test_prefill_splits_only_where_the_partials_pay(tokens, start, splits, monke
     shape = _lib.PrefillShape(tokens, start, 32, 8, 128, 36, 16, 3, _lib.LK_BF16, _lib.LK_BF16, 128**-0.5)
     expected = 0 if splits == 1 else 32 * tokens * splits * 130 * 4
     assert _lib.load().lk_paged_prefill_workspace(shape) == expected
+
+
+@pytest.mark.parametrize("kv,batch,width,splits", [("bf16", 1, 16, 1), ("bf16", 1, 17, 3), ("bf16", 12, 44, 1), ("bf16", 5, 44, 6), ("bf16", 24, 112, 1),
+                                                   ("bf16", 23, 112, 2), ("bf16", 24, 113, 2), ("bf16", 3, 375, 10), ("fp8", 24, 94, 1),
+                                                   ("fp8", 8, 94, 4), ("fp8", 64, 112, 1), ("bf16", 64, 113, 2)])
+def test_decode_short_tables_stay_one_split_where_the_rows_fill_the_gpu(kv, batch, width, splits):
+    """Both sides of the one-split rule's lines, and splits that give a CU no second workgroup (256 CUs)."""
+    from layover_amd.kernels import _lib
+
+    kv_format = _lib.LK_BF16 if kv == "bf16" else _lib.LK_FP8_RECORD
+    shape = _lib.DecodeShape(batch, 32, 8, 128, 36, 16, 0, width, _lib.LK_BF16, kv_format, 1.0 / math.sqrt(128), 0, 0)
+    assert _lib.load().lk_paged_decode_workspace(shape) == batch * 32 * 130 * 4 * splits
