@@ -25,8 +25,9 @@
 //   convert (exact), the group's power of two folded into the score (K) and the weights (V).
 //   Groups whose shift could leave BF16's normal range use the exact integer decode of
 //   fp8.py instead, so results equal attention over the reference's decode_bits output.
-// Generic path (any slots <= 64 and head_dim <= 256, any G): one wave per (sequence, query
-//   head, split), lane d owning dims d, d+64, ...; used for shapes other than Qwen3's.
+// Other shapes: decode_split_tiles (decode_tiles.h) takes every head_dim that is a multiple of 8.
+// Generic path (any G, head_dim <= 256): one wave per (sequence, query head, split),
+//   lane d owning dims d, d+64, ...; for the head_dims left over and pools of odd alignment.
 // Combine: one wave per (sequence, query head) merges the split partials (m, l, acc) and
 //   writes the output rounded to nearest even. A table of one split needs no merge: the
 //   split kernel (8-wave form) writes the output itself. (Merging inside the split kernel,
