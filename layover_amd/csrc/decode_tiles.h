@@ -22,7 +22,7 @@
 // Measured on MI355X, per layer, against one wave per (sequence, query head, split) walking its
 // tokens one at a time (decode_split_generic, which keeps head_dims that are no multiple of 8 and
 // odd alignments): FP32 pool, 32 query heads of 128 dims, batch 4 at 700-2,500 tokens 517 -> 19 us
-// (3.4 TB/s of K and V); BF16, 64 dims, batch 16 at 300-6,000 tokens 908 -> 25 us (3.9 TB/s), the
+// (3.4 TB/s of K and V); BF16, 64 dims, batch 16 at 300-6,000 tokens 908 -> 22 us (4.5 TB/s), the
 // merge launch apart. About 6 us of that is the chain from the launch to the first tile and from
 // the last to the partials; at long contexts the loads set the pace.
 #ifndef LAYOVER_AMD_DECODE_TILES_H
