@@ -36,9 +36,6 @@ namespace lk {
 
 constexpr uint32_t kTilesMaxDim = 256;
 
-// Stands for a zero part of a weight (see the weights' parts below): 2^-120 of a value is nothing.
-constexpr float kTinyPart = 7.52316385e-37f;
-
 // A row of zeros, as long as the longest row (256 FP32 dims).
 static __device__ __align__(16) const uint32_t zero_row[kTilesMaxDim] = {};
 
@@ -243,7 +240,9 @@ __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 :
 #pragma unroll
     for (uint32_t e = 0; e < kVDims; ++e) o[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    auto consume = [&](Tile& tile, uint32_t i) __attribute__((always_inline)) {
+    // kProducts: PV in FP32 products of the whole weights (see the second pass below).
+    auto consume = [&](Tile& tile, uint32_t i, auto products) __attribute__((always_inline)) {
+        constexpr bool kProducts = kF32 || decltype(products)::value;
         const uint32_t token0 = kTileTokens * (wave + i * waves);
         // K and V as FP32 words or BF16 pairs. FP8 codes become BF16 unscaled, or (any shift of the
         // tile out of the plain range: a wave-uniform branch) are decoded with their shifts.
@@ -348,7 +347,7 @@ __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 :
             p[r] *= v_factor[r];
         }
 
-        if constexpr (kF32) {
+        if constexpr (kProducts) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -357,8 +356,7 @@ __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 :
                     o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], value, o[e], 0, 0, 0);
                 }
         } else {
-            // The weights as three BF16 parts, cut (not rounded) from the top, so that no part is
-            // negative, and none zero: with an infinite V every part gives the same infinity.
+            // The weights as three BF16 parts, cut (not rounded) from the top: exact, and none negative.
             uint32_t part[3][2];
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
@@ -366,15 +364,15 @@ __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 :
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
                     part[k][half] = __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
-                    x0 = fmaxf(x0 - bf16_lo(part[k][half]), kTinyPart);
-                    x1 = fmaxf(x1 - bf16_hi(part[k][half]), kTinyPart);
+                    x0 -= bf16_lo(part[k][half]);
+                    x1 -= bf16_hi(part[k][half]);
                 }
             }
-            const uint32_t tiny = __float_as_uint(kTinyPart) | __float_as_uint(kTinyPart) >> 16;
-            // Both steps are the same instruction: a dependent pair of different ones (16x16x32, then
-            // 16x16x16 on its result) lost the first one's product on MI355X.
+            // Both steps are the same instruction: with 16x16x16 on the result of 16x16x32 the first
+            // step's product was missing from the sum (no wait states stand between the two in the
+            // assembly; the cause was not established).
             const bf16x8 p_top = as_bf16x8(part[0][0], part[0][1], part[1][0], part[1][1]);
-            const bf16x8 p_low = as_bf16x8(part[2][0], part[2][1], tiny, tiny);
+            const bf16x8 p_low = as_bf16x8(part[2][0], part[2][1], 0u, 0u);
 #pragma unroll
             for (uint32_t e = 0; e < kVDims; ++e) {
                 const uint32_t select = (e & 1) ? 0x07060302u : 0x05040100u;
@@ -397,8 +395,28 @@ __global__ __launch_bounds__(kD == 256 && (KV == LK_F32 || QF == LK_F32) ? 256 :
         for (uint32_t i = 0; i < mine; i += kRing) {
 #pragma unroll
             for (int d = 0; d < kRing; ++d) {
-                if (i + d < mine) consume(ring[d], i + d);
+                if (i + d < mine) consume(ring[d], i + d, std::false_type{});
                 fetch(ring[d], i + d + kRing);
+            }
+        }
+    }
+    // Zero parts of a weight (its low ones often are, and half of p_low is) make NaN of an infinite V, where
+    // the weight itself makes the infinity: BF16 pools with a NaN in a sum take their tiles again, as
+    // products in FP32, and a NaN that stays is the result's own. (FP8 codes hold no infinity.)
+    if constexpr (!kF32 && KV == LK_BF16) {
+        bool nan = false;
+#pragma unroll
+        for (uint32_t e = 0; e < kVDims; ++e)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) nan = nan || o[e][r] != o[e][r];
+        if (__builtin_expect(__any(nan), 0)) {
+            m = -INFINITY;
+            l = 0.0f;
+#pragma unroll
+            for (uint32_t e = 0; e < kVDims; ++e) o[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (uint32_t i = 0; i < mine; ++i) {
+                fetch(ring[0], i);
+                consume(ring[0], i, std::true_type{});
             }
         }
     }

@@ -97,3 +97,65 @@ def test_tiled_fp8_decode_of_far_shifts_is_exact(exponent):
     # BF16 rounding of the result; below FP32's normals each of the 300 terms may be lost whole.
     scale = np.abs(oracle.bf16_to_float(bits)[:, 1]).max()
     assert (np.abs(got - expected) <= 2.0**-8 * np.abs(expected) + 2.0**-16 * scale + 300 * 2.0**-126).all()
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp32"])
+@pytest.mark.parametrize("head_dim,slots", [(64, 16), (40, 5), (128, 8), (256, 16)])
+def test_tiled_weights_meet_values_of_any_size(kv, head_dim, slots):
+    """A weight that underflows to zero hides a V near BF16's largest value, one of about 2^-104 scales a V
+    of 2^104 to about 1, and an infinity in a visible row comes out as that infinity, whatever the
+    weight it meets."""
+    length = 333
+    width = -(-length // slots)
+    rng = np.random.default_rng(head_dim)
+    # All of a token's K equal kappa and q is all ones: scores are kappa sqrt(head_dim), in nats.
+    nats = 0.5 * rng.standard_normal(width * slots).astype(np.float32)
+    hidden, small, infinite, small_infinite = 40, 100, 200, 310  # tokens
+    nats[hidden], nats[small], nats[small_infinite] = -320.0, -72.0, -72.0
+    k = np.repeat((nats / np.sqrt(head_dim))[:, None], head_dim, axis=1)
+    v = rng.standard_normal((width * slots, head_dim)).astype(np.float32)
+    v[hidden] = 2.0**127
+    v[small] = 2.0**104
+    v[infinite, 0], v[infinite, head_dim - 1] = np.inf, -np.inf
+    v[small_infinite, 3] = -np.inf
+    pool = np.zeros((width, 2, 3, 2, slots, head_dim), dtype=np.float32)
+    for kind, rows in enumerate((k, v)):
+        pool[:, kind, 1] = rows.reshape(width, 1, slots, head_dim)
+    bits, q = oracle.bf16_bits(pool), oracle.bf16_bits(np.ones((1, 4, head_dim), dtype=np.float32))
+    table, lens = np.arange(width, dtype=np.int32).reshape(1, width), np.array([length], dtype=np.int32)
+    expected = oracle.decode_attention(q, bits, 1, table, lens, 2)
+    assert np.isinf(expected[..., [0, 3, head_dim - 1]]).all() and np.isfinite(np.delete(expected, [0, 3, head_dim - 1], axis=-1)).all()
+    got = _run(_bf16(q), _bf16(bits) if kv == "bf16" else _bf16(bits).float(), table, lens, 2)
+    infinities = np.isinf(expected)
+    assert np.array_equal(got[infinities], expected[infinities])
+    # BF16 rounding of the result and FP32 arithmetic as above; the small weight's own error is 2^-24 of
+    # its exponent, about 104.
+    error, size = np.abs(got[~infinities] - expected[~infinities]), np.abs(expected[~infinities])
+    assert (error <= 2.0**-8 * size + 2.0**-24 * 4 * (head_dim + 64)).all(), error.max()
+
+
+@pytest.mark.parametrize("kv,offset", [("bf16", 2), ("fp32", 1), ("fp8", 4)])
+@pytest.mark.parametrize("head_dim,slots,groups", [(24, 16, 2), (64, 16, 4), (128, 8, 16)])
+def test_tiled_decode_of_4_byte_aligned_pools_and_queries(kv, offset, head_dim, slots, groups):
+    """Pools and queries that start 4 bytes past a 16-byte boundary give the same bits."""
+    from layover_amd.kernels.hip_decode import Fp8KVPool
+
+    def shifted(tensor, elements):
+        room = torch.empty(tensor.numel() + elements, dtype=tensor.dtype, device="cuda")
+        view = room[elements:].view(tensor.shape)
+        view.copy_(tensor)
+        assert view.data_ptr() % 16 == 4
+        return view
+
+    q, bits, table, lens = _case(head_dim, slots, groups, [1, 40, 1300], seed=head_dim)
+    if kv == "fp8":
+        ids = np.arange(bits.shape[0])
+        records = torch.from_numpy(oracle.quantize_records(bits, ids, slots * head_dim, 12).reshape(len(ids), -1)).cuda()
+        pools = [Fp8KVPool(r, 3, 2, slots, head_dim) for r in (records, shifted(records, offset))]
+    else:
+        pool = _bf16(bits) if kv == "bf16" else _bf16(bits).float()
+        pools = [pool, shifted(pool, offset)]
+    for q_gpu, q_offset in ((_bf16(q), 2), (_bf16(q).float(), 1)):
+        expected = _run(q_gpu, pools[0], table, lens, groups)
+        assert np.isfinite(expected).all()
+        assert np.array_equal(_run(shifted(q_gpu, q_offset), pools[1], table, lens, groups), expected)
