@@ -352,9 +352,11 @@ void launch_decode(const DecodeArgs& a, const Geometry& g, int kv, void* out, hi
     } else {
         const uint64_t grid = uint64_t(a.batch) * a.query_heads * g.splits;
         require(grid <= 0x7FFFFFFFull, "decode grid too large");
-        if (kv == LK_BF16) hipLaunchKernelGGL((decode_split_generic<LK_BF16, QF>), dim3(uint32_t(grid)), dim3(kWave), 0, stream, a);
-        else if (kv == LK_F32) hipLaunchKernelGGL((decode_split_generic<LK_F32, QF>), dim3(uint32_t(grid)), dim3(kWave), 0, stream, a);
-        else hipLaunchKernelGGL((decode_split_generic<LK_FP8_RECORD, QF>), dim3(uint32_t(grid)), dim3(kWave), 0, stream, a);
+        // A launch holds fewer than 2^32 threads.
+        const dim3 block(kWave * (grid < (1ull << 32) / (kWave * kGenericWaves) ? kGenericWaves : 1));
+        if (kv == LK_BF16) hipLaunchKernelGGL((decode_split_generic<LK_BF16, QF>), dim3(uint32_t(grid)), block, 0, stream, a);
+        else if (kv == LK_F32) hipLaunchKernelGGL((decode_split_generic<LK_F32, QF>), dim3(uint32_t(grid)), block, 0, stream, a);
+        else hipLaunchKernelGGL((decode_split_generic<LK_FP8_RECORD, QF>), dim3(uint32_t(grid)), block, 0, stream, a);
     }
     if (a.out != nullptr) return;  // the split kernel wrote the output
     const dim3 grid(a.batch * a.query_heads, a.layer_count);
