@@ -293,11 +293,11 @@ lk_decode_shape one_layer(const lk_decode_shape& s, uint32_t at) {
 
 // Workspace: split partials, acc [layers, batch, query_heads, splits, head_dim] then (m, l) pairs. Several
 // layers run as one launch, or (with no token write, or shapes and pools the matrix-core kernel does
-// not take) one after the other in the same space.
+// not take) one after the other in the same space: always so for the tiled kernel's shapes.
 uint64_t workspace_bytes(const lk_decode_shape& s) {
-    const uint64_t bytes = partial_bytes(s, geometry(s).splits);
-    if (layer_count(s) == 1) return bytes;
-    return std::max(bytes, workspace_bytes(one_layer(s, 0)));
+    if (layer_count(s) == 1) return partial_bytes(s, geometry(s).splits);
+    const uint64_t apart = workspace_bytes(one_layer(s, 0));
+    return tiled_shape(s) ? apart : std::max(apart, partial_bytes(s, geometry(s).splits));
 }
 
 // Waves per workgroup of the matrix-core kernel: 4 when the grid gives the CUs two or more

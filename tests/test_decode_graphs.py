@@ -319,3 +319,24 @@ def test_decode_short_tables_stay_one_split_where_the_rows_fill_the_gpu(kv, batc
     kv_format = _lib.LK_BF16 if kv == "bf16" else _lib.LK_FP8_RECORD
     shape = _lib.DecodeShape(batch, 32, 8, 128, 36, 16, 0, width, _lib.LK_BF16, kv_format, 1.0 / math.sqrt(128), 0, 0)
     assert _lib.load().lk_paged_decode_workspace(shape) == batch * 32 * 130 * 4 * splits
+
+
+@pytest.mark.parametrize("head_dim,layers_held", [(64, 1), (128, 8)])
+def test_layers_that_run_one_by_one_need_one_layers_workspace(head_dim, layers_held):
+    """A launch of 8 layers holds every layer's partials where the layers run together (16 slots x 128
+    dims), and one layer's where they run one after the other; a captured step is one call either way."""
+    from layover_amd.kernels import _lib
+
+    def need(flags):
+        shape = _lib.DecodeShape(4, 32, 8, head_dim, 8, 16, 0, 256, _lib.LK_BF16, _lib.LK_BF16, 0.1, 0, 0, flags)
+        return _lib.load().lk_paged_decode_workspace(shape)
+
+    assert need(0) > 4 * 32 * (head_dim + 2) * 4  # several splits
+    if layers_held == 1:
+        assert need(8 << 8 | 4 << 16) == need(0)
+    else:
+        assert need(8 << 8 | 4 << 16) > need(0)
+    cfg = ModelConfig(num_hidden_layers=8, num_attention_heads=32, num_key_value_heads=8, head_dim=head_dim)
+    graphs = DecodeAttentionGraphs(PagedKVCache(cfg, 260, fill=False), 32, sizes=(4,), max_tokens=4096, capture=stub_capture)
+    assert graphs._layers_per_launch == {(4, 64): 8, (4, 128): 8, (4, 256): 8}
+    assert graphs._workspaces[4, 256].numel() == max(need(8 << 8 | 4 << 16), *(graphs._workspace_need(4, w) for w in (64, 128)))
