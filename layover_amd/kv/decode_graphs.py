@@ -103,7 +103,7 @@ class DecodeAttentionGraphs:
         kv_dtype = torch.bfloat16 if isinstance(self.pool, Fp8KVPool) else self.pool.dtype
         self.k_new = torch.zeros(self.layers, largest, self.kv_heads, self.head_dim, dtype=kv_dtype, device=device)
         self.v_new = torch.zeros_like(self.k_new)
-        self._rows_used = 0  # rows of q, k_new and v_new from here on hold zeros
+        self._rows_used = 0  # of q, k_new and v_new; from here on their rows hold zeros (see `run`)
         # Table widths captured for every size: the full width and its halvings down to 64
         # blocks. The kernel's split geometry follows the table's width (the lengths are only
         # on the device), so a short batch in a wide table would pay for splits that hold
@@ -173,12 +173,17 @@ class DecodeAttentionGraphs:
         """Replay the captured step of `size` rows and `width` table columns (the full width by
         default) on the buffers as they stand; returns the output tensor that every replay of
         this size and width refreshes."""
-        replay = self._replays[size, width or self.width]
+        self._rows_used = self.sizes[-1]  # the caller may have filled any of them
+        return self._replay(size, width or self.width)
+
+    def _replay(self, size: int, width: int) -> torch.Tensor:
+        replay = self._replays[size, width]
         replay()
         return replay.out
 
     def step_eager(self, size: int, width: int | None = None) -> torch.Tensor:
         """The same step launched eagerly on the same buffers, for comparison."""
+        self._rows_used = self.sizes[-1]
         return self._step(size, width or self.width)
 
     def size_for(self, batch: int) -> int | None:
@@ -201,11 +206,16 @@ class DecodeAttentionGraphs:
         batch = len(tables)
         rows = torch.cat([self.cache.decode_rows(tables, self.width), self._padding(size - batch)])
         self.packed[:size].copy_(rows.to(self.packed.device), non_blocking=True)
+        # Padding rows are zero; the fills are left out where the rows hold zeros already: not since a larger
+        # batch used them, a step was launched on the buffers as they stood (replay, step_eager), or
+        # a call ended between the copies.
+        used = self._rows_used
+        self._rows_used = max(batch, used)
         for buffer, values in ((self.q, q), (self.k_new, k_new), (self.v_new, v_new)):
             buffer[:, :batch].copy_(values)
-            if batch < min(size, self._rows_used):  # padding rows stay zero unless a larger batch used them
+            if batch < min(size, used):
                 buffer[:, batch:size].zero_()
-        self._rows_used = batch if size >= self._rows_used else max(batch, self._rows_used)
-        out = self.replay(size, width)
+        self._rows_used = batch if size >= used else max(batch, used)
+        out = self._replay(size, width)
         # The graph refreshes the same tensor on its next replay.
         return out[:, :batch].clone()

@@ -100,6 +100,33 @@ def test_graphs_decline_batches_and_tables_they_were_not_captured_for():
     assert graphs.run([BlockTable([1, 2, 3], 40)], q[:, :1], kv[:, :1], kv[:, :1]) is None
 
 
+@pytest.mark.parametrize("left_by", ["a_failed_call", "replay", "step_eager"])
+def test_padding_rows_are_zero_after_calls_that_left_other_rows(left_by, monkeypatch):
+    """Rows of q that a call filled before it failed, and rows of all inputs that a caller filled itself for
+    replay or step_eager, are zeros again where the next step pads."""
+    from layover_amd.kv.decode_graphs import Replay
+
+    monkeypatch.setattr(DecodeAttentionGraphs, "_step", lambda self, size, width: None)
+    cache = PagedKVCache(ModelConfig.micro(), 12, fill=False)
+    graphs = DecodeAttentionGraphs(cache, 4, sizes=(2, 4), max_tokens=32,
+                                   capture=lambda step, pool=None: Replay(lambda: None, torch.zeros(2, 4, 4, 24), pool))
+    free = [b for b in range(12) if b not in graphs.scratch_blocks]
+    tables = [BlockTable(free[i : i + 1], i + 1) for i in range(4)]
+    q, kv = torch.ones(2, 4, 4, 24), torch.ones(2, 4, 2, 24)
+    graphs.run(tables[:1], q[:, :1], kv[:, :1], kv[:, :1])
+    if left_by == "a_failed_call":
+        with pytest.raises(RuntimeError):
+            graphs.run(tables, q, kv[:, :3], kv)
+    else:
+        for buffer in (graphs.q, graphs.k_new, graphs.v_new):
+            buffer.fill_(2.0)
+        getattr(graphs, left_by)(4)
+    graphs.run(tables[:1], q[:, :1], kv[:, :1], kv[:, :1])
+    graphs.run(tables[:3], q[:, :3], kv[:, :3], kv[:, :3])
+    for buffer in (graphs.q, graphs.k_new, graphs.v_new):
+        assert bool((buffer[:, :3] == 1).all()) and not buffer[:, 3:].any()
+
+
 def test_graphs_refuse_a_head_count_that_does_not_divide():
     with pytest.raises(ValueError, match="divide"):
         DecodeAttentionGraphs(PagedKVCache(ModelConfig.micro(), 4, fill=False), 3, capture=stub_capture)
