@@ -740,7 +740,7 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
     };
 
     PrefillStaged staged;
-    // One step: set 0's scores, then set 1's beside set 0's exponentials, set 0's PV beside set 1's
+    // One step (BF16): set 0's scores, then set 1's beside set 0's exponentials, set 0's PV beside set 1's
     // exponentials, set 1's PV: the wave's VALU work always has independent MFMAs beside it. The
     // scheduling barrier after set 0's scores keeps the two sets' QK products from being mixed, which
     // would leave set 0's softmax nothing to run beside. Then the next step's tiles go into the other
@@ -770,17 +770,28 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
         values(step, vb);
         f32x4 s[2][2];
         scores(0, kk, s[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        // Raised wave priority from here to the end of set 1's PV: the SIMD's other wave is then mostly in a
-        // matrix-core stretch, whose MFMAs keep running while this wave's dependent chain is issued
-        // first. From set 0's scores on 985 us per layer on the long chunk, from here 940, after set
-        // 1's scores 1,001, never 1,025 (same box; the priority instruction also keeps what stands
-        // before it from being scheduled past it); lowered before set 1's PV 868 against 865 there, 84.2
-        // against 82.9 us on the 509-token chunk.
-        __builtin_amdgcn_s_setprio(1);
-        scores(1, kk, s[1]);
+        float top[2];  // FP8
+        if constexpr (KV == LK_BF16) {
+            __builtin_amdgcn_sched_barrier(0);
+            // Raised wave priority from here to the end of set 1's PV: the SIMD's other wave is then mostly in a
+            // matrix-core stretch, whose MFMAs keep running while this wave's dependent chain is issued
+            // first. From set 0's scores on 985 us per layer on the long chunk, from here 940, after set
+            // 1's scores 1,001, never 1,025 (same box; the priority instruction also keeps what stands
+            // before it from being scheduled past it); lowered before set 1's PV 868 against 865 there, 84.2
+            // against 82.9 us on the 509-token chunk.
+            __builtin_amdgcn_s_setprio(1);
+            scores(1, kk, s[1]);
+            if constexpr (kMasked) mask(step, 0, s[0]);
+        } else {
+            // FP8 pools: both sets' scores, then the softmax stretch of both at raised priority, with set
+            // 0's PV in between; the BF16 order above, on MI355X, 512 tokens at 4,000 and 2,048 at 8,203
+            // (8 KV heads x 4) 185 and 464 us -> 196 and 486.
+            scores(1, kk, s[1]);
+            if constexpr (kMasked) mask(step, 0, s[0]);
+            __builtin_amdgcn_s_setprio(1);
+            top[0] = lane_max(s[0], f);
+        }
         if constexpr (kMasked) {
-            mask(step, 0, s[0]);
             mask(step, 1, s[1]);
             // Keys at or past the chunk's end hold anything: zero their V (0 * NaN is NaN).
             const uint32_t key0 = step * 2 * kSlots;
@@ -813,8 +824,7 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
                 if (set == 1) __builtin_amdgcn_s_setprio(0);
             }
         } else {
-            __builtin_amdgcn_s_setprio(1);
-            const float top[2] = {lane_max(s[0], f), lane_max(s[1], f)};
+            top[1] = lane_max(s[1], f);
             rescale(top);
             const bf16x8 p0 = weights(0, s[0], f);
             accumulate(0, p0, vb);
