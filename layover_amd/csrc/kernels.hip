@@ -149,7 +149,7 @@ uint64_t pool_block_bytes(const lk_decode_shape& s) {
 // The matrix-core kernel needs the Qwen3 tile shape (16 slots x 128 dims), at most 16 query
 // heads per KV head, a BF16 or FP8-record pool, 16-byte aligned tiles (pool base and block
 // stride) and blocks below 2 GiB (its loads address a block through a buffer resource of 32-bit
-// size); anything else runs the generic kernel.
+// size). The tiled kernel takes most other shapes (tiled_decode), the generic one the rest.
 bool fast_decode(const lk_decode_shape& s, const void* pool) {
     const uint32_t groups = s.query_heads / s.kv_heads;
     return s.slots == kSlots && s.head_dim == kDim && groups <= kMaxHeads && s.kv_format != LK_F32 && aligned(pool, 16) &&
@@ -304,13 +304,32 @@ uint64_t workspace_bytes(const lk_decode_shape& s) {
 // workgroups each; otherwise 8 (at most 8 query heads per KV head), so the few workgroups
 // still put two waves on each SIMD. (16 waves would leave each 128 registers, and the kernel
 // needs more.) LAYOVER_DECODE_WAVES=4|8 forces a count the head group allows.
-uint32_t decode_waves(const DecodeArgs& a, uint64_t grid) {
-    const uint32_t forced = env_waves();
-    if (forced == 4 || (forced == 8 && a.groups <= 8)) return forced;
-    // Short tables: 8 waves write the outputs of a row's only split themselves.
-    if (a.splits == 1 && a.groups <= 8) return 8;
-    if (grid >= 2ull * compute_units()) return 4;
-    return a.groups <= 8 ? 8 : 4;
+// Tables of one split: 8 waves write the outputs themselves, which saves the merge launch, on larger
+// grids too, until they keep more CUs waiting than that saves: later for wide tables, and for BF16, whose
+// chains of loads gain from twice the waves. Measured on MI355X per layer, 4 query heads per KV head, rows of
+// one length, with 4 waves and with 8:
+//   FP8, 32 blocks, 3 and 4 workgroups per CU 25.3 and 32.5, 26.9 and 34.8 us; 112 blocks, 2, 3 and 4 per
+//   CU 44.7, 63.6 and 83.2, 43.9, 64.7 and 84.9 (one row of 112 blocks beside rows of 14: 25.9, 27.9 and
+//   30.0, 18.7, 23.3 and 28.4)
+//   BF16, 64 blocks, 4 and 8 per CU 83.4 and 158.4, 79.0 and 153.3 us; 1 query head per KV head with the
+//   token write, 4 blocks, 4 per CU 15.9 and 18.6
+//   FP8 with the token write, whose 8 waves leave room for one workgroup on a CU, 32 blocks, 2 and 3 per CU
+//   23.0 and 28.9, 25.2 and 35.7; 112 blocks, 2 per CU 52.3 and 51.3
+uint32_t decode_waves(const lk_decode_shape& s, uint32_t splits, uint64_t grid, bool append) {
+    const uint32_t forced = env_waves(), groups = s.query_heads / s.kv_heads;
+    const uint64_t cus = compute_units();
+    const bool fp8 = s.kv_format == LK_FP8_RECORD;
+    if (forced == 4 || (forced == 8 && groups <= 8)) return forced;
+    if (groups > 8) return 4;
+    if (splits == 1) {
+        const uint32_t width = s.table_width;
+        uint64_t per_cu = 0;  // workgroups up to which 8 waves are faster
+        if (fp8 && append) per_cu = width > 64 ? 2 : 0;
+        else if (fp8) per_cu = width > 64 ? 4 : (width > 32 ? 3 : 2);
+        else per_cu = width > 64 ? 8 : (width > 32 || groups >= 4 ? 4 : 2);
+        if (grid <= per_cu * cus) return 8;
+    }
+    return grid >= 2 * cus ? 4 : 8;
 }
 
 template <int KV, int QF, bool kAppend>
@@ -721,17 +740,17 @@ void run_decode(const lk_decode_shape& s, const void* q, const void* pool, const
     a.bps = g.bps;
     a.layer_count = layer_count(s);
     a.layer_rows = layer_rows(s);
-    a.waves = decode_waves(a, uint64_t(s.batch) * a.layer_count * g.splits * s.kv_heads);
+    a.waves = decode_waves(s, g.splits, uint64_t(s.batch) * a.layer_count * g.splits * s.kv_heads, write != nullptr);
     a.order = env_order();
     a.shared_blocks = (s.flags & LK_DECODE_SHARED_BLOCKS) != 0;
     a.vector_combine = aligned(workspace, 16) && aligned(out, s.q_format == LK_BF16 ? 8 : 16);
     a.slots_inverse = s.slots > 1 ? uint32_t(((1ull << 32) + s.slots - 1) / s.slots) : 0;
     a.block_bytes = pool_block_bytes(s);
     a.scale_log2 = s.scale * kLog2e;
-    // One split per row (tables of at most `bps` blocks) on a grid small enough for 8-wave
-    // workgroups: the split kernel writes the output. (The 4-wave kernel has no such branch,
-    // which measurably costs the large-batch loop.) LAYOVER_DECODE_COMBINE keeps the combine
-    // launch (for comparisons).
+    // One split per row (tables of at most `bps` blocks): the split kernel writes the output, the
+    // matrix-core one where it runs with 8 waves (see decode_waves; its 4-wave form has no such
+    // branch, which measurably costs the large-batch loop), the tiled one always.
+    // LAYOVER_DECODE_COMBINE keeps the combine launch (for comparisons).
     if (g.fast && g.splits == 1 && env_combine() == 0 && a.waves == 8) a.out = out;
     if (g.tiled && g.splits == 1 && env_combine() == 0) a.out = out;
     require(aligned(pool, s.kv_format == LK_F32 ? 4 : (s.kv_format == LK_BF16 ? 2 : 1)), "misaligned pool");

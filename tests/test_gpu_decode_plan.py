@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("kv", ["bf16", "fp8"])
-@pytest.mark.parametrize("batch,width", [(1, 16), (1, 17), (5, 13), (12, 44), (24, 112), (23, 112), (24, 113), (3, 375), (70, 90)])
+@pytest.mark.parametrize("batch,width", [(1, 16), (1, 17), (5, 13), (12, 44), (24, 112), (23, 112), (24, 113), (3, 375), (70, 90), (65, 30), (97, 33), (130, 60), (260, 66)])
 def test_decode_across_the_split_plan(batch, width, kv):
     from layover_amd.kernels import fp8, hip_decode
 
