@@ -772,10 +772,9 @@ __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(K
 // Generic path: one workgroup per (sequence, query head, split), whose waves take a contiguous run of
 // the split's tokens each and meet in LDS; lane d owns dims d, d + 64, ... A wave's tokens are one
 // dependent chain (load, dot product, shuffles, exponential), so the waves in flight set the pace.
-// Eight of them, whatever split plan the launch follows, are faster than one wave a split was with more
-// and shorter splits: measured on MI355X per layer, 32 query heads of 100 dims over 8 KV heads, 1, 16 and 32
-// rows of 512 tokens 91, 322 and 634 us as 4, 2 and 1 splits of one wave, 52, 100 and 107 us as one
-// split of eight (four: 95, 182 and 192); 32 rows of 2,048 tokens 1,351 us as 2, 395 us as one.
+// Measured on MI355X per layer, 32 query heads of 100 dims over 8 KV heads, 1, 16 and 32 rows of 512 tokens in 4, 2
+// and 1 splits of one wave 91, 322 and 634 us, in one split of eight waves 52, 100 and 107 (four: 95, 182 and
+// 192), in the splits of generic_bps (kernels.hip) 17, 53 and 105.
 
 template <int KV>
 __device__ __forceinline__ float kv_element(const uint8_t* tile, uint32_t index, int32_t shift) {
@@ -792,11 +791,16 @@ template <int KV, int QF>
 __global__ __launch_bounds__(kWave* kGenericWaves) void decode_split_generic(DecodeArgs a) {
     __shared__ float s_acc[kGenericWaves][kMaxGenericDim], s_ml[kGenericWaves][2];
     const uint32_t waves = blockDim.x / kWave, wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const uint32_t split = blockIdx.x % a.splits;
-    const uint32_t pair = blockIdx.x / a.splits;
-    const uint32_t qh = pair % a.query_heads;
-    const uint32_t seq = pair / a.query_heads;
-    const uint32_t kv_head = qh / a.groups;
+    // KV head fastest, then the query head of its group, the sequence, the split: the query heads that read
+    // the same tokens share an XCD wherever there are a multiple of 8 KV heads, the heads of a row longer
+    // than the others spread over CUs, and the first splits, which hold all the tokens of short rows, over XCDs. Measured on MI355X, 100 dims, 8 splits: one
+    // row of 8,192 tokens beside 31 of 1,024, 1,454 us with the split fastest, 353 so; 32 rows of 8,192 1,450
+    // and 1,436, and 1,570 with the query heads of a KV head side by side.
+    const uint32_t pairs = a.batch * a.query_heads;
+    const uint32_t split = blockIdx.x / pairs;
+    const uint32_t seq = blockIdx.x % pairs / a.query_heads;
+    const uint32_t kv_head = blockIdx.x % a.query_heads % a.kv_heads;
+    const uint32_t qh = kv_head * a.groups + blockIdx.x % a.query_heads / a.kv_heads;
     const int32_t length = a.lengths[uint64_t(seq) * a.lengths_stride];
     const uint32_t nblocks = blocks_of(length, a.slots);
     const uint32_t first = split * a.bps;

@@ -169,7 +169,8 @@ bool tiled_decode(const lk_decode_shape& s, const void* q, const void* pool) {
 uint32_t layer_count(const lk_decode_shape& s) { return std::max((s.flags >> 8) & 0xFFu, 1u); }
 uint32_t layer_rows(const lk_decode_shape& s) { return s.flags >> 16; }
 
-// Whether a shape belongs to the tiled kernel; misaligned pools of other shapes use its plan too.
+// Whether a shape belongs to the tiled or the generic kernel; misaligned pools of the tiled kernel's shapes
+// use its plan too.
 bool tiled_shape(const lk_decode_shape& s) {
     return !(s.slots == kSlots && s.head_dim == kDim && s.kv_format != LK_F32 && s.query_heads / s.kv_heads <= kMaxHeads);
 }
@@ -211,6 +212,20 @@ TiledPlan tiled_plan(const lk_decode_shape& s) {
     tiles = std::max(tiles, units * width / 65536);
     p.bps = uint32_t(std::min<uint64_t>((tiles * kTileTokens + s.slots - 1) / s.slots, 256));
     return p;
+}
+
+// Blocks per split of the generic kernel (head_dims that are no multiple of 8): about four workgroups of
+// 8 waves per CU, which is all the waves it holds, of 64 to 1,024 tokens. Measured on
+// MI355X per layer, BF16, 32 query heads of 100 dims over 8 KV heads, 16 slots: 1 and 16 rows of 512 tokens 17.5
+// and 53 us in 8 and 2 splits, 56 and 105 in one (the tiled kernel's plan); 250 dims, 8 slots, 4 rows of 512
+// tokens 28 us in 8, 179 in one; 100 dims, 32 rows of 8,192 tokens, splits of 256, 512, 1,024 and 2,048
+// tokens 1,507, 1,469, 1,458 and 1,501 us.
+uint32_t generic_bps(const lk_decode_shape& s) {
+    const uint64_t rows = uint64_t(s.batch) * s.query_heads, width = uint64_t(s.table_width) * s.slots;
+    const uint64_t splits = std::max<uint64_t>(4ull * compute_units() / rows, 1);
+    uint64_t tokens = std::min<uint64_t>(std::max<uint64_t>((width + splits - 1) / splits, 64), 1024);
+    tokens = std::max(tokens, rows * width / 65536);  // as many workgroups as the largest launches should have at most
+    return uint32_t(std::min<uint64_t>((tokens + s.slots - 1) / s.slots, 256));
 }
 
 Geometry geometry(const lk_decode_shape& s, const void* pool = nullptr) {
@@ -256,11 +271,10 @@ Geometry geometry(const lk_decode_shape& s, const void* pool = nullptr) {
         }
         if (tiled_shape(s)) {
             // Partials that lk_paged_decode_static can hold, as long as 64-block splits or larger keep them so.
-            uint32_t tiled = tiled_plan(s).bps;
+            bps = s.head_dim % 8 == 0 ? tiled_plan(s).bps : generic_bps(s);
             uint64_t most = 64;
             while (most < large && most < 256) most *= 2;
-            while (tiled < most && partial_bytes(s, (s.table_width + tiled - 1) / tiled) > kStaticScratchBytes) ++tiled;
-            bps = tiled;
+            while (bps < most && partial_bytes(s, (s.table_width + bps - 1) / bps) > kStaticScratchBytes) ++bps;
         }
     }
     g.bps = bps;

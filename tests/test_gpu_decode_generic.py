@@ -15,7 +15,9 @@ LAYERS, HEADS = 3, 2
 # head_dim, slots, groups, lengths, whether in several splits; pools of the last shapes start one element past alignment.
 SHAPES = [
     (31, 16, 4, [1, 3, 17, 3000], True),
-    (31, 7, 1, [2, 500], False),
+    (31, 7, 1, [2, 500], True),
+    (31, 7, 1, [2, 63], False),
+    (255, 16, 2, [30, 64], False),
     (100, 16, 4, [5, 700, 2049], True),
     (100, 200, 2, [199, 200, 201, 1500], True),
     (255, 4, 3, [9, 1333], True),
