@@ -68,10 +68,17 @@ bool fast_records(const void* pool, const void* stage, uint64_t group_elems, uin
 }
 
 // The vector kernels take what 16-byte loads of the pool and 8-byte ones of the records (4-byte aligned)
-// can: every even number of groups a block of a multiple of 8 values, up to 4,096.
-bool vector_records(const void* pool, const void* stage, uint32_t count, uint64_t group_elems, uint32_t groups_per_block) {
+// can: every even number of groups a block of a multiple of 8 values, up to 4,096. Small totals of small
+// groups (side by side, or half of a wave's lanes) stay with the element loops, a wave for each group, where a
+// vector wave's many groups are one chain: up to 4,096 groups, of 384 values and 2^20 in all for quantize, 128
+// and 2^19 for dequantize. Measured on MI355X, elements and vector: quantize 3,072 groups of 128, 256 and 384 values
+// 4.2, 4.8 and 5.5, 4.8, 5.2 and 5.0 us, 1,800 of 256 and 384 4.4 and 4.9, 5.4 and 5.1, 24,576 of 128 10.8 and
+// 5.8; dequantize 3,072 of 128 and 256 3.7 and 4.1, 4.0 and 3.8.
+bool vector_records(const void* pool, const void* stage, uint32_t count, uint64_t group_elems, uint32_t groups_per_block, bool quantize) {
+    const uint64_t total = uint64_t(count) * groups_per_block, values = total * group_elems;
+    if (total <= 4096 && group_elems <= (quantize ? 384u : 128u) && values < (quantize ? 1u << 20 : 1u << 19)) return false;
     return group_elems % 8 == 0 && group_elems <= kVectorGroup && groups_per_block % 2 == 0 && aligned(pool, 16) && aligned(stage, 4) &&
-           uint64_t(count) * groups_per_block < 0x7FFFFFFFull;
+           total < 0x7FFFFFFFull;
 }
 
 // Decode launch geometry: blocks per split (bps) and splits per sequence, from the shape only.
@@ -593,7 +600,7 @@ LK_EXPORT int lk_fp8_quantize(const void* pool, const int32_t* ids, uint32_t cou
         if (lk::fast_records(pool, stage, group_elems, groups_per_block))
             lk::launch_quantize_2048(static_cast<const uint16_t*>(pool), ids, static_cast<uint8_t*>(stage), count, groups_per_block,
                                      lk::codec_grid(groups), s);
-        else if (lk::vector_records(pool, stage, count, group_elems, groups_per_block))
+        else if (lk::vector_records(pool, stage, count, group_elems, groups_per_block, true))
             lk::launch_quantize_vector(static_cast<const uint16_t*>(pool), ids, static_cast<uint8_t*>(stage), uint32_t(groups),
                                        uint32_t(group_elems), groups_per_block, s);
         else
@@ -614,7 +621,7 @@ LK_EXPORT int lk_fp8_dequantize(const void* stage, const int32_t* ids, uint32_t 
         if (lk::fast_records(pool, stage, group_elems, groups_per_block))
             lk::launch_dequantize_2048(static_cast<const uint8_t*>(stage), ids, static_cast<uint16_t*>(pool), count, groups_per_block,
                                        lk::codec_grid(groups), s);
-        else if (lk::vector_records(pool, stage, count, group_elems, groups_per_block))
+        else if (lk::vector_records(pool, stage, count, group_elems, groups_per_block, false))
             lk::launch_dequantize_vector(static_cast<const uint8_t*>(stage), ids, static_cast<uint16_t*>(pool), uint32_t(groups),
                                          uint32_t(group_elems), groups_per_block, s);
         else
