@@ -71,25 +71,40 @@ bool any_pair_divides(const lk_prefill_shape& s, uint64_t row_tiles, int32_t bia
     return false;
 }
 
-// Microseconds of a launch whose tiles run `splits` ways, from what the kernel measured on MI355X: a start
-// and an end of 6.5 us, 0.6 us a step for a workgroup alone on its CU, 0.78 for two that share one,
-// whole rounds of two per CU beyond that; and the merge, a launch (3 us) over partials written and read
-// at 5 TB/s. Model and measurement (8 KV heads x 4, us per layer): 391 tokens at 0 in 1, 2 and 3 splits
-// 14.3, 18.9, 22.6 and 14.3, 20.8, 23.7; 509 at 8,203 in 2 and 4 98, 76 and 96, 75; 1,000 at 1,000 in 1
-// and 2 44, 48 and 44, 47; 64 at 4,000 in 8 and 31 22, 26 and 23, 26. Splitting until every CU had two
-// workgroups, whatever the partials cost, took 23.7, 75, 47 and 26 us there, and 82 us for 1,900 tokens
-// at 300 (480 workgroups, short of 512) where one way takes 47.
-double split_cost(const lk_prefill_shape& s, uint32_t cus, uint64_t row_tiles, uint32_t steps, uint32_t splits) {
-    const uint64_t workgroups = row_tiles * s.kv_heads * splits, rounds = (workgroups + 2 * cus - 1) / (2 * cus);
-    const uint32_t groups = s.query_heads / s.kv_heads;
-    double each = (steps + splits - 1) / splits;
-    if (splits == 1 && workgroups > cus) {
-        // Heavy and light tiles share CUs (PrefillArgs::paired) and, where they differ, their steps.
-        const uint32_t light = lds_tile_steps(s.start, uint64_t(s.tokens) * groups, groups, 0);
-        each = std::min<double>(each, (steps + light + kPairBias) / 2.0 + 4.0);
+// Row tiles of the largest chunk that may split its keys: below two workgroups for each of 256 CUs.
+constexpr uint64_t kPlanTiles = 512;
+
+// Microseconds of a launch whose tiles run `wanted` ways, from what the kernel measured on MI355X: 12 us
+// around the first 8 steps of a chain, 0.67 us a further step of a workgroup that has its CU to itself, 0.82 of
+// one that shares it (0.88 for unsplit chains, whose light tiles end early), again for every further round of
+// two per CU, the last by what is left of it; and the merge, 2.5 us over partials written and read at 4.2 TB/s,
+// and 0.2 for each split past the 8 whose loads it issues at once. Workgroups whose split starts past their
+// tile's keys end at once and are not counted; unsplit pairs of tiles divide their steps (any_pair_divides)
+// whether they share a CU or not. Measured (us per layer, the splits chosen, and those that filled two
+// workgroups per CU whatever the partials cost): 4 query heads on each of 8 KV heads, 391 tokens at 0 in 1 and 3
+// 17.2 and 26.1, 509 at 8,203 in 4 82, 64 at 4,000 in 10 and 26 23.9 and 28.9, 1,900 at 300 in 1 and 2 49 and
+// 84; 1 query head on each, 2,300 at 1,500 in 3 and 4 51 and 64, 2,700 at 3,000 and 1,900 at 0 in 3 and 1 71
+// and 32, in the 2 that a model without empty workgroups and undivided tiles took 91 and 36.
+double split_cost(const lk_prefill_shape& s, uint32_t cus, const uint32_t* tile_steps, uint64_t tiles, uint32_t wanted) {
+    const uint32_t longest = tile_steps[tiles - 1], split_steps = (longest + wanted - 1) / wanted;
+    const uint32_t splits = (longest + split_steps - 1) / split_steps;
+    // Splits are dealt to XCDs and shader engines in turn, four or eight of them, so an even number of splits
+    // leaves some of these with the first splits of every tile, which all hold keys.
+    const uint32_t turn = splits % 4 == 0 ? 4 : (splits % 2 == 0 ? 2 : 1);
+    uint64_t workgroups = 0;
+    for (uint64_t tile = 0; tile < tiles; ++tile) {
+        const uint32_t live = (tile_steps[tile] + split_steps - 1) / split_steps;
+        workgroups += (live + turn - 1) / turn * turn;
     }
-    double cost = 6.5 + each * (workgroups <= cus ? 0.6 : 0.78) * rounds;
-    if (splits > 1) cost += 3.0 + 2.0 * s.query_heads * double(s.tokens) * splits * (kDim + 2) * sizeof(float) / 5e6;
+    workgroups *= s.kv_heads;
+    const double chain = splits > 1 ? split_steps : std::min<double>(longest, (longest + tile_steps[0] + kPairBias) / 2.0 + 2.0);
+    const double shared = splits > 1 ? 0.82 : 0.88;
+    const uint64_t full = workgroups / (2 * cus), rest = workgroups % (2 * cus);
+    double cost = 12.0 + (chain - 8.0) * (shared * full + (rest == 0 ? 0.0 : rest <= cus ? 0.67 : shared));
+    if (splits > 1) {
+        cost += 2.5 + 2.0 * s.query_heads * double(s.tokens) * splits * (kDim + 2) * sizeof(float) / 4.2e6;
+        if (splits > 8) cost += 0.2 * (splits - 8);
+    }
     return cost;
 }
 
@@ -119,13 +134,16 @@ PrefillPlan prefill_plan(const lk_prefill_shape& s) {
         wanted = uint32_t(strtoul(forced, nullptr, 10));
     } else {
         const uint64_t workgroups = p.row_tiles * s.kv_heads, target = 2ull * compute_units();
-        if (workgroups < target) {
-            const uint64_t fill = (target + workgroups - 1) / workgroups;
+        if (workgroups < target && p.row_tiles <= kPlanTiles) {
+            // Up to one split more than gives every CU two workgroups, of at least 4 steps.
+            const uint64_t fill = (target + workgroups - 1) / workgroups + 1;
             const uint32_t cap = uint32_t(std::min<uint64_t>({fill, max_steps / 4, kMaxKeySplits}));
+            uint32_t tile_steps[kPlanTiles];
+            for (uint64_t tile = 0; tile < p.row_tiles; ++tile) tile_steps[tile] = lds_tile_steps(s.start, rows, groups, tile);
             wanted = 1;
-            double least = split_cost(s, uint32_t(target / 2), p.row_tiles, max_steps, 1);
+            double least = split_cost(s, uint32_t(target / 2), tile_steps, p.row_tiles, 1);
             for (uint32_t n = 2; n <= cap; ++n) {
-                const double cost = split_cost(s, uint32_t(target / 2), p.row_tiles, max_steps, n);
+                const double cost = split_cost(s, uint32_t(target / 2), tile_steps, p.row_tiles, n);
                 if (cost < least) {
                     least = cost;
                     wanted = n;

@@ -348,6 +348,23 @@ def test_decode_short_tables_stay_one_split_where_the_rows_fill_the_gpu(kv, batc
     assert _lib.load().lk_paged_decode_workspace(shape) == batch * 32 * 130 * 4 * splits
 
 
+@pytest.mark.parametrize("groups,tokens,start,splits", [(4, 509, 8203, 4), (4, 1, 300, 2), (4, 64, 4000, 10), (4, 1700, 30000, 2), (1, 2300, 1500, 3),
+                                                        (1, 3000, 1000, 3), (4, 17, 0, 1), (4, 1900, 300, 1), (1, 1900, 0, 1)])
+def test_prefill_splits_follow_the_work_that_each_way_leaves(groups, tokens, start, splits):
+    """Splits that hold no keys of their tile, divided tiles and the merge's bytes count (256 CUs, 8 KV heads); partials
+    of [KV heads, rows, splits] of 128 values and (m, l)."""
+    from layover_amd.kernels import _lib
+
+    shape = _lib.PrefillShape(tokens, start, 8 * groups, 8, 128, 2, 16, 1, _lib.LK_BF16, _lib.LK_BF16, 0.1)
+    need = _lib.load().lk_paged_prefill_workspace(shape)
+    row_bytes = 8 * groups * tokens * 130 * 4
+    if splits > 1:
+        assert need == -(-row_bytes * splits // 256) * 256
+    else:  # divided tiles only: 80 floats a thread for each side of a pair of tiles, and two words
+        pairs = 8 * ((-(-tokens * groups // 128) + 1) // 2)
+        assert need in (0, -(-pairs * 2 * 256 * 80 * 4 // 256) * 256 + -(-pairs * 16 // 256) * 256)
+
+
 @pytest.mark.parametrize("head_dim,layers_held", [(64, 1), (128, 8)])
 def test_layers_that_run_one_by_one_need_one_layers_workspace(head_dim, layers_held):
     """A launch of 8 layers holds every layer's partials where the layers run together (16 slots x 128
