@@ -125,8 +125,8 @@ struct DecodeArgs {
     uint32_t write_stride;
     const uint16_t* k_new;
     const uint16_t* v_new;
-    // Non-null when every row fits one split (splits == 1, matrix-core kernel with 8 waves):
-    // that split's state is the answer, so the split kernel writes the output here and no
+    // Non-null when every row fits one split and the kernel can write outputs (the matrix-core one with 8
+    // waves, the tiled one): that split's state is the answer, so the split kernel writes the output here and no
     // combine runs.
     void* out;
 };

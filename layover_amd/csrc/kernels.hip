@@ -259,8 +259,8 @@ Geometry geometry(const lk_decode_shape& s, const void* pool = nullptr) {
     //     65 -> 53.5 us; FP8 at 1,500, batch 24 and 64: 24.6 -> 15.6, 41.7 -> 32.4; batch 12 even). A
     //     row that is much longer than the others is one workgroup's chain, so the line is not
     //     drawn where even rows alone would have it (BF16 at 3,000, batch 32: 61 -> 53 us).
-    //   Rows of one launch's several layers stay split above 64 blocks (three rows of 600-2,000
-    //   tokens x 36 layers: 192 us a step in 64-block splits, 204 in one).
+    //   Rows of one launch's several layers go by the other two rules, whose splits hold 64 blocks where the
+    //   layers fill the GPU (three rows of 600-2,000 tokens x 36 layers: 170 us a step so, 184 in one split).
     uint32_t bps = env_bps() > 256 ? 256 : env_bps();
     if (bps == 0) {
         const uint64_t work = units * s.table_width, width = s.table_width, cus = compute_units();

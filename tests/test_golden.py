@@ -169,7 +169,7 @@ def assert_attention_close(out, expected, weighted_abs_v=None):
         allowed = allowed + 2.0**-8 * weighted_abs_v
     assert np.isfinite(got).all()
     assert (np.abs(got - expected) <= allowed).all(), np.abs(got - expected).max()
-    assert (np.abs(got - expected) <= 2e-2 + 1e-2 * np.abs(expected)).all()  # north-star tolerance
+    assert (np.abs(got - expected) <= 2e-2 + 1e-2 * np.abs(expected)).all()
 
 
 @pytest.mark.gpu

@@ -11,7 +11,8 @@ from oracle import oracle
 pytestmark = pytest.mark.gpu
 
 # head_dim, slots, groups, lengths: class edges (8/32/40/64/72/128/136/256 dims), tiles that end
-# inside a block and blocks inside a tile, more than 16 query heads (two chunks), rows of one token.
+# inside a block and blocks inside a tile, more than 16 query heads (two chunks), rows of one token, the
+# matrix-core kernel's shape with the pools that it does not take (FP32, unaligned records).
 SHAPES = [
     (8, 16, 1, [1, 16, 33]),
     (24, 16, 2, [1, 384, 2300]),
@@ -22,6 +23,7 @@ SHAPES = [
     (72, 24, 5, [23, 700]),
     (128, 16, 20, [1, 130, 1100]),
     (128, 8, 16, [7, 8, 9, 2050]),
+    (128, 16, 4, [33, 3100, 5000]),
     (136, 16, 2, [47, 260]),
     (256, 16, 9, [1, 2100]),
     (256, 64, 1, [63, 64, 65, 900]),

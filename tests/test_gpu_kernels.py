@@ -1,7 +1,7 @@
 """GPU parity of the HIP kernels against the CPU oracle, through the C ABI wrappers.
 
 FP8: bit-exact (every BF16 pattern x every shift the computed scale can produce, and whole
-records at the Qwen3-4B and micro shapes). Decode: within the north-star tolerance
+records at the Qwen3-4B and micro shapes). Decode: within the tolerance
 (2e-2 abs / 1e-2 rel at BF16) of the float64 oracle, and much tighter in practice: the
 asserted bound is the BF16 rounding of the exact answer plus a small FP32 allowance.
 """
@@ -232,7 +232,7 @@ def weighted_mean_abs_v(q, pool_bits, layer, table, lengths, groups):
 def assert_close_to_oracle(out, expected, what="", weight_rounding=None):
     got = out.double().cpu().numpy()
     # BF16 rounding of the exact answer (2^-8 relative) plus an FP32 accumulation allowance;
-    # far inside the north-star 2e-2 abs / 1e-2 rel. weight_rounding: the weighted mean of
+    # far inside 2e-2 abs / 1e-2 rel. weight_rounding: the weighted mean of
     # |v| where the kernel feeds the weights to the matrix cores as single BF16s (FP8 pools).
     allowed = np.abs(expected) * 2.0**-8 + 1e-3
     if weight_rounding is not None:
@@ -322,12 +322,12 @@ def test_decode_fp8_pool_matches_the_oracle_on_the_dequantized_pool(fp8, hip_dec
     fp8_pool = hip_decode.Fp8KVPool(torch.from_numpy(records.reshape(blocks, -1)).cuda(), layers, kv_heads, slots, head_dim)
     out = hip_decode.paged_decode_attention_hip(to_gpu_bf16(q), fp8_pool, 2, torch.from_numpy(table).cuda(), torch.from_numpy(lens).cuda(), 4)
     # The aligned records run the matrix-core kernel, whose FP8 path rounds the weights to
-    # BF16; the unaligned ones the generic FP32 kernel.
+    # BF16; the unaligned ones the tiled kernel, whose weights keep 24 bits.
     rounding = weighted_mean_abs_v(q, dequantized, 2, table, lens, 4) if layers == 4 else None
     assert_close_to_oracle(out, expected, "fp8 records", weight_rounding=rounding)
 
 
-@pytest.mark.parametrize("layers", [4, 1], ids=["fast_kernel", "generic_kernel"])
+@pytest.mark.parametrize("layers", [4, 1], ids=["fast_kernel", "tiled_kernel"])
 def test_decode_fp8_pool_with_extreme_shifts_uses_the_exact_decode(fp8, hip_decode, layers):
     kv_heads, slots, head_dim = 2, 16, 128
     q, pool, table, lens = decode_case([40], layers, kv_heads, slots, head_dim, groups=2, seed=10)

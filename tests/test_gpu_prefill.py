@@ -1,6 +1,6 @@
 """Paged causal prefill (lk_paged_prefill) against the float64 oracle, through the C ABI.
 
-Tolerance: the north star's 2e-2 absolute / 1e-2 relative, plus a tighter check that the
+Tolerance: 2e-2 absolute / 1e-2 relative, plus a tighter check that the
 error stays within BF16 rounding of the output and of the weights (P enters the matrix cores
 as BF16): |err| <= 2^-7 |x| + 4e-3."""
 
@@ -286,7 +286,7 @@ def test_prefill_gives_the_same_bits_on_every_launch(start, tokens, kv_heads, gq
     """Six launches of the same chunk give identical outputs bit for bit. A maximum written as
     inline assembly once read matrix-core results without the wait states the compiler
     inserts for its own instructions: the second 16 rows of a wave then varied from launch
-    to launch (still within the north-star tolerance), at GQA 3-5 with two or more key steps."""
+    to launch (still within the tolerance), at GQA 3-5 with two or more key steps."""
     from layover_amd.kernels.hip_prefill import paged_prefill_attention_hip
 
     end = start + tokens

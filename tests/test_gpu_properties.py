@@ -3,7 +3,7 @@
 The first follows the reference's own property test (tests/test_triton_decode.py:335-353):
 the same strategy space (1-3 KV heads, GQA 1/2/4, head dims 8-32 including odd ones, 4/7/16
 slots, layers 0-2, q gains 0.1-8, BF16 or FP32, 1-4 rows of 1-70 tokens), which here runs
-the generic kernel. The second draws the Qwen3 tile shape (16 slots x 128 dims), which runs
+the tiled kernel, and the generic one for 31 dims. The second draws the Qwen3 tile shape (16 slots x 128 dims), which runs
 the matrix-core kernel, over BF16 pools and FP8 records, 1-40 rows of up to 3,000 tokens.
 The third draws FP8 record layouts, alignments and counts for the swap's record kernels.
 Draws are derandomized, so every run checks the same cases.
@@ -37,7 +37,7 @@ def make_case(lengths, kv_heads, groups, head_dim, slots, layers, seed, gain, po
 def assert_close(out, expected, weighted_abs_v=None):
     """BF16 rounding of the exact answer plus an FP32 allowance (and, for FP8 records, whose
     weights reach the matrix cores as single BF16s, 2^-8 of the attention-weighted mean |v|),
-    inside the north-star 2e-2 abs / 1e-2 rel."""
+    inside 2e-2 abs / 1e-2 rel."""
     got = out.double().cpu().numpy()
     allowed = np.abs(expected) * 2.0**-8 + 1e-3
     if weighted_abs_v is not None:
