@@ -98,7 +98,8 @@ typedef struct {
  * hold every layer's queries at once. Table and lengths (and write positions) serve all of them; q
  * and k, v of layer i start at row i * rows of the arrays given (rows >= batch, below 65536), out is
  * [count, batch, query_heads, head_dim] contiguous. The same results as one call per layer, up to
- * the order in which a row's partial sums are added; the workspace is sized for the whole launch.
+ * the order in which a row's partial sums are added; the workspace is sized for the layers that run
+ * at once (all where the matrix-core kernel takes the shape, one elsewhere).
  * Not for lk_paged_decode_static. */
 #define LK_DECODE_LAYERS(count, rows) (((uint32_t)(count) << 8) | ((uint32_t)(rows) << 16))
 

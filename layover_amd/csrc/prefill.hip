@@ -80,11 +80,11 @@ constexpr uint64_t kPlanTiles = 512;
 // two per CU, the last by what is left of it; and the merge, 2.5 us over partials written and read at 4.2 TB/s,
 // and 0.2 for each split past the 8 whose loads it issues at once. Workgroups whose split starts past their
 // tile's keys end at once and are not counted; unsplit pairs of tiles divide their steps (any_pair_divides)
-// whether they share a CU or not. Measured (us per layer, the splits chosen, and those that filled two
-// workgroups per CU whatever the partials cost): 4 query heads on each of 8 KV heads, 391 tokens at 0 in 1 and 3
-// 17.2 and 26.1, 509 at 8,203 in 4 82, 64 at 4,000 in 10 and 26 23.9 and 28.9, 1,900 at 300 in 1 and 2 49 and
-// 84; 1 query head on each, 2,300 at 1,500 in 3 and 4 51 and 64, 2,700 at 3,000 and 1,900 at 0 in 3 and 1 71
-// and 32, in the 2 that a model without empty workgroups and undivided tiles took 91 and 36.
+// whether they share a CU or not. Measured (us per layer in the splits chosen, and in as many as give every CU two
+// workgroups): 4 query heads on each of 8 KV heads, 391 tokens at 0 in 1 and 3 18.0 and 25.5, 64 at 4,000 in 10
+// and 26 23.7 and 28.6, 1,000 at 1,000 in 1 and 2 47.6 and 51.9, 1,900 at 300 in 1 and 2 56 and 94; 1 query head
+// on each, 2,500 at 1,000 in 3 and 4 52 and 62, 3,000 at 1,000 in 3 57 (69 in 2, which counting empty
+// workgroups and undivided tiles would choose), 1,900 at 0 in 1 and 5 31.4 and 32.6 (36.1 in 2).
 double split_cost(const lk_prefill_shape& s, uint32_t cus, const uint32_t* tile_steps, uint64_t tiles, uint32_t wanted) {
     const uint32_t longest = tile_steps[tiles - 1], split_steps = (longest + wanted - 1) / wanted;
     const uint32_t splits = (longest + split_steps - 1) / split_steps;
