@@ -47,7 +47,7 @@ struct PrefillPlan {
 // Steps moved toward the heavy side of a divided tile (the partner side pays a second
 // prologue and epilogue); LAYOVER_PREFILL_PAIR_BIAS overrides it, read per launch. Measured on
 // MI355X, 2,048 tokens at position 0 (partner on the heavy remainder first): 0.049-0.051 ms per
-// layer at 8, 0.049 at 10, 0.050-0.051 at 12, 0.050-0.052 at 14-16 (two runs each, one box).
+// layer at 8, 0.049 at 10, 0.050-0.051 at 12, 0.050-0.052 at 14-16 (two runs each, one card).
 // The staggered step (prefill_attention.h) moved the optimum a little: 40.7, 40.5, 40.9 and 41.1 us at 6,
 // 8, 10 and 12.
 constexpr int32_t kPairBias = 8;

@@ -342,7 +342,7 @@ __global__ __launch_bounds__(kWave* kPrefillWaves) void prefill_mfma(PrefillArgs
 // sums on the matrix cores; 1.13 ms with the lane-local rescale check; 1.10 ms with the
 // direct-to-LDS copies two steps ahead into the swizzled layout. Steps in pairs with one
 // barrier per pair (four buffers) against a barrier per step (three): 1.064-1.077 -> 1.059-1.067
-// ms there (on a slower box), and 0.060-0.062 -> 0.058 ms for a 2,048-token chunk at position 0.
+// ms there (on a slower card), and 0.060-0.062 -> 0.058 ms for a 2,048-token chunk at position 0.
 // O leaves through LDS: its rows are spread over lanes by dim (16e + n), so each wave writes
 // its 32 rows there and reads them back as 16-byte pieces of whole rows.
 constexpr uint32_t kLdsWaves = 4;
@@ -746,11 +746,11 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
     // would leave set 0's softmax nothing to run beside. Then the next step's tiles go into the other
     // buffer and the one after into registers. Steps that need the causal mask (and the chunk-end V
     // mask, which only the last step can need) run in a second copy of the loop.
-    // Measured on MI355X (A/B on one box, 2,048 tokens ending a 32,768 context, 2,048 at 0, and 509 at
+    // Measured on MI355X (A/B on one card, 2,048 tokens ending a 32,768 context, 2,048 at 0, and 509 at
     // 8,203 of an FP8 pool): 951, 42.2 and 90.0 us per layer with the maxima of both sets ahead of any
     // exponential; 926, 41.3 and 88.0 with the check on the weights; 877, 40.8 and 84.9 with the sets
     // staggered. On top of that: MFMAs and VALU work dealt one to 2, 3 or 4 by scheduling groups 959,
-    // 943 and 959 against 940 us on another box; K of the next step read ahead of set 1's PV 934 us
+    // 943 and 959 against 940 us on another card; K of the next step read ahead of set 1's PV 934 us
     // against 877 (its registers spill the loop's); the weight sums by dot products of the packed pairs
     // instead of the MFMA against ones 922 against 875: VALU slots are as scarce as matrix ones.
     auto run_step = [&](uint32_t step, auto masked_tag) __attribute__((always_inline)) {
@@ -776,7 +776,7 @@ __global__ __launch_bounds__(kWave* kLdsWaves) __attribute__((amdgpu_waves_per_e
             // Raised wave priority from here to the end of set 1's PV: the SIMD's other wave is then mostly in a
             // matrix-core stretch, whose MFMAs keep running while this wave's dependent chain is issued
             // first. From set 0's scores on 985 us per layer on the long chunk, from here 940, after set
-            // 1's scores 1,001, never 1,025 (same box; the priority instruction also keeps what stands
+            // 1's scores 1,001, never 1,025 (same card; the priority instruction also keeps what stands
             // before it from being scheduled past it); lowered before set 1's PV 868 against 865 there, 84.2
             // against 82.9 us on the 509-token chunk.
             __builtin_amdgcn_s_setprio(1);
