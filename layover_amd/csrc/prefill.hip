@@ -142,7 +142,7 @@ PrefillPlan prefill_plan(const lk_prefill_shape& s) {
             for (uint64_t tile = 0; tile < p.row_tiles; ++tile) tile_steps[tile] = lds_tile_steps(s.start, rows, groups, tile);
             wanted = 1;
             double least = split_cost(s, uint32_t(target / 2), tile_steps, p.row_tiles, 1);
-            for (uint32_t n = 2; n <= cap; ++n) {
+            for (uint32_t n = 2; n <= cap; n += 1 + n / 16) {  // many splits differ little, and each costs host time
                 const double cost = split_cost(s, uint32_t(target / 2), tile_steps, p.row_tiles, n);
                 if (cost < least) {
                     least = cost;
