@@ -365,6 +365,16 @@ def test_prefill_splits_follow_the_work_that_each_way_leaves(groups, tokens, sta
         assert need in (0, -(-pairs * 2 * 256 * 80 * 4 // 256) * 256 + -(-pairs * 16 // 256) * 256)
 
 
+@pytest.mark.parametrize("head_dim,slots,batch,tokens,splits", [(100, 16, 1, 512, 8), (100, 16, 16, 512, 2), (100, 16, 32, 512, 1), (250, 8, 4, 512, 8),
+                                                               (31, 16, 1, 64, 1), (31, 64, 2, 4096, 16), (100, 16, 64, 8192, 8)])
+def test_generic_decode_splits_for_workgroups_not_for_kv_heads(head_dim, slots, batch, tokens, splits):
+    """head_dims that are no multiple of 8: about four workgroups per CU (256 CUs, 32 query heads), of 64 to 1,024 tokens."""
+    from layover_amd.kernels import _lib
+
+    shape = _lib.DecodeShape(batch, 32, 8, head_dim, 2, slots, 0, tokens // slots, _lib.LK_BF16, _lib.LK_BF16, 0.1, 0, 0)
+    assert _lib.load().lk_paged_decode_workspace(shape) == batch * 32 * (head_dim + 2) * 4 * splits
+
+
 @pytest.mark.parametrize("head_dim,layers_held", [(64, 1), (128, 8)])
 def test_layers_that_run_one_by_one_need_one_layers_workspace(head_dim, layers_held):
     """A launch of 8 layers holds every layer's partials where the layers run together (16 slots x 128
